@@ -345,6 +345,65 @@ __device__ __forceinline__ bool row_part(const Csr& csr, int64_t n, int part, in
   return beg < end;
 }
 
+// Row, share and CSR range of a wave in the kernels that sum over a row's segment: `slots` row slots of
+// `parts` waves each (consecutive waves of one block).  valid is false past the last slot or for a
+// traversal entry outside the rows; the wave then has an empty range.
+struct RowShare {
+  int64_t n;
+  int32_t beg, end;
+  int wave, part;   // of the block, of the row
+  bool valid;
+};
+__device__ __forceinline__ RowShare row_share(const Csr& csr, int64_t wave, int64_t slots, int64_t rows, int parts) {
+  RowShare r;
+  const int64_t slot = parts == 1 ? wave : wave / parts;
+  r.wave = (int)(wave & (kWavesPerBlock - 1));
+  r.part = r.wave & (parts - 1);
+  r.n = slot < slots ? visit_row(csr, slot, rows) : -1;
+  r.valid = r.n >= 0;
+  r.beg = r.end = 0;
+  if (r.valid) {
+    if (parts == 1) {
+      r.beg = csr.ptr[r.n];
+      r.end = csr.ptr[r.n + 1];
+    } else if (!row_part(csr, r.n, r.part, parts, r.beg, r.end)) {
+      r.end = r.beg;
+    }
+  }
+  return r;
+}
+
+// A row's sum over its CSR segment split over `parts` waves of one block (1, 2 or 4: sum_parts in
+// ictc_launch.h): each wave sums one share, then the shares are added in part order through LDS, a slice of
+// kSumSlice components at a time, and each of the row's waves stores every parts-th component.  Every wave
+// of the block calls this (barriers inside); `valid` is false for waves without a row, and they only keep
+// the barriers.  parts == 1: the plain row store, no LDS and no barrier.
+constexpr int kSumSlice = 12;
+template <int N>
+__device__ __forceinline__ void store_row_sum(float* __restrict__ base, int C, int c, float* v, int parts,
+                                              const RowShare& rs, bool valid) {
+  if (parts == 1) {
+    if (valid && c < C) store_row<N>(base, C, c, v);
+    return;
+  }
+  __shared__ float share[kWavesPerBlock][kSumSlice][kWave];
+  const int w = rs.wave, part = rs.part, w0 = w - part, l = c & (kWave - 1);
+#pragma unroll
+  for (int k0 = 0; k0 < N; k0 += kSumSlice) {
+    const int n = N - k0 < kSumSlice ? N - k0 : kSumSlice;
+#pragma unroll
+    for (int k = 0; k < kSumSlice; ++k)
+      if (k0 + k < N) share[w][k][l] = v[k0 + k];
+    __syncthreads();
+    for (int k = part; k < n; k += parts) {
+      float t = share[w0][k][l];
+      for (int q = 1; q < parts; ++q) t += share[w0 + q][k][l];
+      if (valid && c < C) base[(int64_t)(k0 + k) * C + c] = t;
+    }
+    __syncthreads();
+  }
+}
+
 // Edge metadata of a chunk of up to 64 consecutive CSR positions, staged one
 // edge per lane with coalesced loads; the edge loop then reads it with
 // readlane (wave-uniform SGPR values, no memory latency inside the loop).
@@ -413,17 +472,17 @@ constexpr bool msg_fwd_pipelined() {
 
 template <class T>
 __global__ __launch_bounds__(kBlock, (Occupancy<kMsgFwd, T::LI, T::LE, T::LO>::value)) void msg_fwd_kernel(
-    Operands a, const int64_t* __restrict__ src, Csr csr, float* __restrict__ out) {
+    Operands a, const int64_t* __restrict__ src, Csr csr, float* __restrict__ out, int parts) {
   const RowGroup rg = row_group_y_xcd();
-  if (rg.row >= a.rows) return;
-  const int64_t n = visit_row(csr, rg.row, a.rows);
-  if (n < 0) return;
+  const RowShare rs = row_share(csr, rg.row, a.rows, a.rows, parts);
+  if (parts == 1 && !rs.valid) return;
+  const int64_t n = rs.n;
+  const int32_t beg = rs.beg, end = rs.end;
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float o[T::NO];
 #pragma unroll
   for (int k = 0; k < T::NO; ++k) o[k] = 0.f;
-  const int32_t beg = csr.ptr[n], end = csr.ptr[n + 1];
   if constexpr (msg_fwd_pipelined<T>()) {
     auto run = [&](auto weighted) {
     constexpr bool W = decltype(weighted)::value;
@@ -465,7 +524,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgFwd, T::LI, T::LE, T::LO>::v
     };
     if (a.weight) run(Flag<true>{});
     else run(Flag<false>{});
-    if (active) store_row<T::NO>(out + n * (int64_t)(T::NO * C), C, c, o);
+    store_row_sum<T::NO>(out + n * (int64_t)(T::NO * C), C, c, o, parts, rs, rs.valid);
     return;
   }
   for (int32_t pos = beg; pos < end; pos += kWave) {
@@ -487,7 +546,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgFwd, T::LI, T::LE, T::LO>::v
       }
     }
   }
-  if (active) store_row<T::NO>(out + n * (int64_t)(T::NO * C), C, c, o);
+  store_row_sum<T::NO>(out + n * (int64_t)(T::NO * C), C, c, o, parts, rs, rs.valid);
 }
 
 // Gate-tangent mode of the first adjoint: per edge, the harmonic gradient (when
@@ -631,17 +690,18 @@ __global__ __launch_bounds__(kBlock, (edge_adjoint_waves<T, TAN>())) void msg_bw
 // Source-owned adjoint: node feature gradient over the source-sorted CSR.
 template <class T>
 __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX, T::LI, T::LE, T::LO>::value)) void msg_bwd_x_kernel(
-    Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx) {
+    Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx,
+    int parts) {
   const RowGroup rg = row_group_y_xcd();
-  if (rg.row >= a.rows) return;
-  const int64_t n = visit_row(scsr, rg.row, a.rows);
-  if (n < 0) return;
+  const RowShare rs = row_share(scsr, rg.row, a.rows, a.rows, parts);
+  if (parts == 1 && !rs.valid) return;
+  const int64_t n = rs.n;
+  const int32_t beg = rs.beg, end = rs.end;
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float d[T::NX];
 #pragma unroll
   for (int i = 0; i < T::NX; ++i) d[i] = 0.f;
-  const int32_t beg = scsr.ptr[n], end = scsr.ptr[n + 1];
   // An out-of-range receiver contributes zero (mask 0, row 0 read).
   for (int32_t pos = beg; pos < end; pos += kWave) {
     const int32_t count = min(end - pos, kWave);
@@ -662,7 +722,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX, T::LI, T::LE, T::LO>::
       }
     }
   }
-  if (active) store_row<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d);
+  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid);
 }
 
 // Source-owned complete adjoint: the feature gradient of each source row and,
@@ -699,21 +759,21 @@ template <class T, bool TAN, bool W = false>
 __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd_src_kernel(
     Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx,
     float* __restrict__ dsh, float* __restrict__ dsh_part, float* __restrict__ dgates, const float* __restrict__ gdot,
-    float* __restrict__ dr, float* __restrict__ dr_part) {
+    float* __restrict__ dr, float* __restrict__ dr_part, int parts) {
   const RowGroup rg = row_group_y_xcd();
-  if (rg.row > a.rows) return;
-  const int64_t n = visit_row(scsr, rg.row, a.rows);
-  if (n < 0) return;
+  const RowShare rs = row_share(scsr, rg.row, a.rows + 1, a.rows, parts);
+  if (parts == 1 && !rs.valid) return;
+  const int64_t n = rs.n;
+  const int32_t beg = rs.beg, end = rs.end;
   const bool tail = n == a.rows;
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float* dsh_g = group_target(dsh, dsh_part, rg.group, a.edges, T::NY);
   float* dr_g = rg.group > 0 ? dr_part + (int64_t)(rg.group - 1) * a.edges : dr;
   float xv[T::NX], d[T::NX];
-  if (active && !tail) load_row<T::NX>(a.x + n * (int64_t)(T::NX * C), C, c, xv);
+  if (active && rs.valid && !tail) load_row<T::NX>(a.x + n * (int64_t)(T::NX * C), C, c, xv);
   else zero_row<T::NX>(xv);
   zero_row<T::NX>(d);
-  const int32_t beg = scsr.ptr[n], end = scsr.ptr[n + 1];
   if constexpr (src_adjoint_pipelined<T, TAN>()) {
     // Two edges in flight: the cotangent, gate and gate-tangent rows of edge i + 1 load while edge i
     // computes (2 waves per SIMD leave room for the second set of rows).  Per-edge arithmetic is that
@@ -770,7 +830,7 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd
     }
     };
     run(Flag<W>{});
-    if (active && !tail && dx) store_row<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d);
+    store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);
     return;
   }
   // An out-of-range receiver contributes zero (mask 0, row 0 read).
@@ -828,7 +888,7 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd
       }
     }
   }
-  if (active && !tail && dx) store_row<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d);
+  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);
 }
 
 // ---------------------------------------------------------------------------

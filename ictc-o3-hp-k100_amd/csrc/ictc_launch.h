@@ -32,7 +32,7 @@ hipError_t launch_msg_fwd(const TpShape& s, const Operands& a, const int64_t* sr
 // Small graphs (cfg2's 4,096 rows) fit the L2 and keep every wave.
 template <class T>
 inline size_t bwd_x_lds_cap(int64_t rows) {
-  return (T::LI == 2 && T::LE == 2 && T::LO == 2 && rows >= 65536) ? 72 * 1024 : 0;
+  return (T::LI == 2 && T::LE == 2 && T::LO == 2 && rows >= 65536) ? 60 * 1024 : 0;   // + the 12 KB of store_row_sum
 }
 
 hipError_t launch_msg_bwd(const TpShape& s, const Operands& a, const int64_t* src, const int64_t* dst, Csr dcsr,
@@ -73,6 +73,23 @@ inline int row_parts(int64_t row_slots, int groups) {
   if (waves <= 0) return 1;
   const int64_t p = (32768 + waves - 1) / waves;
   return (int)(p < 1 ? 1 : (p > 8 ? 8 : p));
+}
+
+// Waves per row (1, 2 or 4, of one block) for the kernels that sum over a row's segment: a small graph does
+// not fill the GPU with one wave per row, and a wave then walks its row's ~40 edges with nothing to hide the
+// loads of the next edge behind.  Measured (us, one wave per row -> split): (2,2,2) C64 on 256 rows
+// msg_fwd 35 -> 15, gate-tangent adjoint 79 -> 32; on 432 rows msg_fwd2 118 -> 43, msg_bwd_x2 76 -> 28;
+// (3,3,3) C64 on 1,359 rows msg_fwd 192 -> 168, msg_bwd_x 228 -> 201.
+// The receiver-owned sums stop there: with two waves per SIMD of rows and more the split costs its partial
+// sums and a second row set-up (4,096 rows msg_fwd 111 -> 115, 16,384 waves msg_fwd2 2,945 -> 3,003).
+// The source-owned adjoints gather the wide receiver cotangent rows, and four waves on one row gather four
+// times fewer distinct rows at once: (2,3,3) C128 on 3,963 rows msg_bwd_x 984 -> 782 (two waves per row 921),
+// (2,2,2) C64 on 4,096 rows all-in-one adjoint 320 -> 297; at 16,384 waves msg_bwd_x 2,595 -> 2,632, so no
+// split from there.
+constexpr int64_t kSumWaves = 4096, kSourceSumWaves = 16384;
+inline int sum_parts(int64_t rows, int groups, int64_t target) {
+  const int64_t waves = rows * groups;
+  return waves >= target ? 1 : (2 * waves >= target ? 2 : 4);
 }
 
 }  // namespace ictc

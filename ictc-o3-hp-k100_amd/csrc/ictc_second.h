@@ -146,16 +146,16 @@ __device__ __forceinline__ void stage_tangent(const float* __restrict__ tsh, con
 // ---------------------------------------------------------------------------
 template <class T>
 __global__ __launch_bounds__(kBlock, (Occupancy<kMsgFwd2, T::LI, T::LE, T::LO>::value)) void msg_fwd2_kernel(
-    Operands a, Tangents t, const int64_t* __restrict__ src, Csr csr, float* __restrict__ out) {
+    Operands a, Tangents t, const int64_t* __restrict__ src, Csr csr, float* __restrict__ out, int parts) {
   const RowGroup rg = row_group_y_xcd();
-  if (rg.row >= a.rows) return;
-  const int64_t n = visit_row(csr, rg.row, a.rows);
-  if (n < 0) return;
+  const RowShare rs = row_share(csr, rg.row, a.rows, a.rows, parts);
+  if (parts == 1 && !rs.valid) return;
+  const int64_t n = rs.n;
+  const int32_t beg = rs.beg, end = rs.end;
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float o[T::NO];
   zero<T::NO>(o);
-  const int32_t beg = csr.ptr[n], end = csr.ptr[n + 1];
   for (int32_t pos = beg; pos < end; pos += kWave) {
     const int32_t count = min(end - pos, kWave);
     Chunk<T> ch;
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgFwd2, T::LI, T::LE, T::LO>::
       }
     }
   }
-  if (active) store_row<T::NO>(out + n * (int64_t)(T::NO * C), C, c, o);
+  store_row_sum<T::NO>(out + n * (int64_t)(T::NO * C), C, c, o, parts, rs, rs.valid);
 }
 
 // Receiver-owned: per-edge harmonic and gate outputs (row `rows` zero-fills the
@@ -281,16 +281,16 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdEdge2, T::LI, T::LE, T::L
 template <class T>
 __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX2, T::LI, T::LE, T::LO>::value)) void msg_bwd_x2_kernel(
     Operands a, Tangents t, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad,
-    float* __restrict__ dx) {
+    float* __restrict__ dx, int parts) {
   const RowGroup rg = row_group_y_xcd();
-  if (rg.row >= a.rows) return;
-  const int64_t n = visit_row(scsr, rg.row, a.rows);
-  if (n < 0) return;
+  const RowShare rs = row_share(scsr, rg.row, a.rows, a.rows, parts);
+  if (parts == 1 && !rs.valid) return;
+  const int64_t n = rs.n;
+  const int32_t beg = rs.beg, end = rs.end;
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float d[T::NX];
   zero<T::NX>(d);
-  const int32_t beg = scsr.ptr[n], end = scsr.ptr[n + 1];
   for (int32_t pos = beg; pos < end; pos += kWave) {
     const int32_t count = min(end - pos, kWave);
     Chunk<T> ch;
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX2, T::LI, T::LE, T::LO>:
       }
     }
   }
-  if (active) store_row<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d);
+  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid);
 }
 
 }  // namespace ictc

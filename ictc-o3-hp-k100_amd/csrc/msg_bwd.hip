@@ -14,12 +14,12 @@ struct MsgBwd {
   hipStream_t st;
   template <class T>
   hipError_t run() {
-    const int G = channel_groups(a.channels);
+    const int G = channel_groups(a.channels), sum = sum_parts(a.rows, G, kSourceSumWaves);
     // One source-owned pass for all three (rows + 1 slots: the last covers the out-of-range tail) where it
     // keeps 2 waves per SIMD; the P17 shapes need the register room of two separate passes.
     if (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value >= 2 && dx && (dsh || dg)) {
-      hipLaunchKernelGGL((msg_bwd_src_kernel<T, false>), dim3(blocks_for(a.rows + 1), G), dim3(kBlock),
-                         0, st, a, dst, scsr, grad, dx, dsh, ws, dg, nullptr, nullptr, nullptr);
+      hipLaunchKernelGGL((msg_bwd_src_kernel<T, false>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
+                         0, st, a, dst, scsr, grad, dx, dsh, ws, dg, nullptr, nullptr, nullptr, sum);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
       if (dsh) return launch_group_sum(dsh, ws, a.edges * T::NY, G - 1, st);
@@ -35,8 +35,8 @@ struct MsgBwd {
       if (dsh && (err = launch_group_sum(dsh, ws, a.edges * T::NY, G - 1, st)) != hipSuccess) return err;
     }
     if (dx) {
-      hipLaunchKernelGGL((msg_bwd_x_kernel<T>), dim3(blocks_for(a.rows), G), dim3(kBlock), bwd_x_lds_cap<T>(a.rows),
-                         st, a, dst, scsr, grad, dx);
+      hipLaunchKernelGGL((msg_bwd_x_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock),
+                         bwd_x_lds_cap<T>(a.rows), st, a, dst, scsr, grad, dx, sum);
       return hipGetLastError();
     }
     return hipSuccess;

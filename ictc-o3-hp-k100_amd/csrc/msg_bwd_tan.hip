@@ -16,16 +16,16 @@ struct MsgBwdTan {
   hipStream_t st;
   template <class T>
   hipError_t run() {
-    const int G = channel_groups(a.channels);
+    const int G = channel_groups(a.channels), sum = sum_parts(a.rows, G, kSourceSumWaves);
     float* ws_dr = ws ? ws + (int64_t)(G - 1) * a.edges * T::NY : nullptr;
     hipError_t err;
     if (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value >= 2 && dx) {
       if (a.weight)
-        hipLaunchKernelGGL((msg_bwd_src_kernel<T, true, true>), dim3(blocks_for(a.rows + 1), G), dim3(kBlock), 0, st,
-                           a, dst, scsr, grad, dx, dsh, ws, nullptr, gdot, dr, ws_dr);
+        hipLaunchKernelGGL((msg_bwd_src_kernel<T, true, true>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
+                           0, st, a, dst, scsr, grad, dx, dsh, ws, nullptr, gdot, dr, ws_dr, sum);
       else
-        hipLaunchKernelGGL((msg_bwd_src_kernel<T, true, false>), dim3(blocks_for(a.rows + 1), G), dim3(kBlock), 0, st,
-                           a, dst, scsr, grad, dx, dsh, ws, nullptr, gdot, dr, ws_dr);
+        hipLaunchKernelGGL((msg_bwd_src_kernel<T, true, false>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
+                           0, st, a, dst, scsr, grad, dx, dsh, ws, nullptr, gdot, dr, ws_dr, sum);
       if ((err = hipGetLastError()) != hipSuccess) return err;
     } else {
       const int parts = row_parts(a.rows + 1, G);
@@ -33,8 +33,8 @@ struct MsgBwdTan {
                          st, a, src, dcsr, grad, dsh, ws, nullptr, parts, gdot, dr, ws_dr);
       if ((err = hipGetLastError()) != hipSuccess) return err;
       if (dx) {
-        hipLaunchKernelGGL((msg_bwd_x_kernel<T>), dim3(blocks_for(a.rows), G), dim3(kBlock),
-                           bwd_x_lds_cap<T>(a.rows), st, a, dst, scsr, grad, dx);
+        hipLaunchKernelGGL((msg_bwd_x_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock),
+                           bwd_x_lds_cap<T>(a.rows), st, a, dst, scsr, grad, dx, sum);
         if ((err = hipGetLastError()) != hipSuccess) return err;
       }
     }

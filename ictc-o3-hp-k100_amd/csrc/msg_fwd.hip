@@ -12,8 +12,9 @@ struct MsgFwd {
   hipStream_t st;
   template <class T>
   hipError_t run() {
-    const int G = channel_groups(a.channels);
-    hipLaunchKernelGGL((msg_fwd_kernel<T>), dim3(blocks_for(a.rows), G), dim3(kBlock), 0, st, a, src, csr, out);
+    const int G = channel_groups(a.channels), parts = sum_parts(a.rows, G, kSumWaves);
+    hipLaunchKernelGGL((msg_fwd_kernel<T>), dim3(blocks_for(a.rows * parts), G), dim3(kBlock), 0, st, a, src, csr, out,
+                       parts);
     return hipGetLastError();
   }
 };

@@ -17,8 +17,9 @@ struct MsgSecondRcv {
   hipError_t run() {
     const int G = channel_groups(a.channels);
     if (dgrad) {
-      hipLaunchKernelGGL((msg_fwd2_kernel<T>), dim3(blocks_for(a.rows), G), dim3(kBlock), 0, st, a, t, src, csr,
-                         dgrad);
+      const int sum = sum_parts(a.rows, G, kSumWaves);
+      hipLaunchKernelGGL((msg_fwd2_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t, src, csr,
+                         dgrad, sum);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
     }

@@ -14,9 +14,9 @@ struct MsgSecondSrc {
   hipStream_t st;
   template <class T>
   hipError_t run() {
-    const int G = channel_groups(a.channels);
-    hipLaunchKernelGGL((msg_bwd_x2_kernel<T>), dim3(blocks_for(a.rows), G), dim3(kBlock), 0, st, a, t, dst, csr, grad,
-                       dx);
+    const int G = channel_groups(a.channels), sum = sum_parts(a.rows, G, kSourceSumWaves);
+    hipLaunchKernelGGL((msg_bwd_x2_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t, dst, csr,
+                       grad, dx, sum);
     return hipGetLastError();
   }
 };
