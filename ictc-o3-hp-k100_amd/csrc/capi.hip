@@ -151,6 +151,159 @@ size_t sort_temp_bytes(int64_t E, int64_t N) {
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
+// ---- Stable counting sort of small key lists --------------------------------
+// The library radix sort takes 8 to 14 launches of about 5 us each below a few hundred thousand keys (a block
+// sort and log2 merge passes), launch-bound throughout.  Here a pass over one 8-bit digit is three launches:
+// per-tile digit counts, one block's scan of [digit][tile], and the scatter, in which a key's place is its
+// digit's scanned base for the tile, plus the counts of the tile's earlier waves, plus that of the wave's
+// earlier keys (ballots of equal digits), so equal digits keep their order.  Up to 255 distinct keys (species
+// ids) one pass sorts and its scan yields ptr; receiver lists of up to 65,535 rows take two.  Measured (us of
+// kernels): 65,000 edges over 1,359 receivers 65 -> 44 and 10 launches -> 7; 8,191 species ids 37 -> 14 and
+// 8 -> 3.
+constexpr int kDigits = 256, kTile = 1024, kSortWaves = 4, kRounds = kTile / (64 * kSortWaves);
+
+// Lanes of the wave with this lane's digit (all 64 lanes call it; an inactive lane passes active = false).
+__device__ __forceinline__ uint64_t same_digit(int d, bool active) {
+  uint64_t m = __ballot(active);
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const uint64_t v = __ballot((d >> b) & 1);
+    m &= ((d >> b) & 1) ? v : ~v;
+  }
+  return m;
+}
+
+// Key of item i: from the caller's int64 keys (out of range -> N, after all others) or the previous pass.
+__device__ __forceinline__ int32_t sort_key(const int64_t* __restrict__ keys, const int32_t* __restrict__ k32,
+                                            int64_t i, int64_t N) {
+  if (k32) return k32[i];
+  const int64_t k = keys[i];
+  return (k >= 0 && k < N) ? (int32_t)k : (int32_t)N;
+}
+
+// hist[w][d]: keys with digit d in the tile's 256-key stretch of wave w.  Every thread of the block calls it.
+__device__ __forceinline__ void tile_histogram(const int64_t* __restrict__ keys, const int32_t* __restrict__ k32,
+                                               int64_t E, int64_t N, int shift, int32_t (*hist)[kDigits],
+                                               int32_t* key, int32_t* rank) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  for (int d = threadIdx.x; d < kSortWaves * kDigits; d += blockDim.x) hist[d / kDigits][d % kDigits] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int64_t i = (int64_t)blockIdx.x * kTile + w * (kTile / kSortWaves) + r * 64 + l;
+    const bool active = i < E;
+    key[r] = active ? sort_key(keys, k32, i, N) : 0;
+    const int d = (key[r] >> shift) & (kDigits - 1);
+    const uint64_t m = same_digit(d, active);
+    const int before = __popcll(m & ((1ull << l) - 1));
+    // the wave alone touches its histogram row: every lane reads its digit's count, then the first of the
+    // equals adds to it (volatile: in this order, and a wave's LDS accesses complete in order)
+    volatile int32_t* h = &hist[w][d];
+    const int32_t seen = active ? *h : 0;
+    rank[r] = seen + before;
+    if (active && before == 0) *h = seen + __popcll(m);
+  }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void sort_count_kernel(const int64_t* __restrict__ keys,
+                                                         const int32_t* __restrict__ k32, int64_t E, int64_t N,
+                                                         int shift, int digits, int32_t* __restrict__ counts) {
+  __shared__ int32_t hist[kSortWaves][kDigits];
+  int32_t key[kRounds], rank[kRounds];
+  tile_histogram(keys, k32, E, N, shift, hist, key, rank);
+  const int d = threadIdx.x;
+  if (d >= digits) return;
+  int32_t t = 0;
+#pragma unroll
+  for (int w = 0; w < kSortWaves; ++w) t += hist[w][d];
+  counts[(int64_t)d * gridDim.x + blockIdx.x] = t;
+}
+
+// Exclusive scan of counts [digits][tiles] in place by one block; with ptr (one pass, digits = N + 1 keys):
+// ptr[n] = base of digit n, ptr[N + 1] = E.
+__global__ __launch_bounds__(1024) void sort_scan_kernel(int32_t* __restrict__ counts, int digits, int tiles,
+                                                         int64_t E, int32_t* __restrict__ ptr) {
+  __shared__ int32_t wave_total[16];
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  // at most 256 * 256 counts; each thread owns `per` groups of four (the array is padded to whole groups of all
+  // threads), loaded 16 bytes at a time
+  const int total = digits * tiles, per = (total + 4095) / 4096;
+  int4* mine4 = (int4*)counts + threadIdx.x * per;
+  const int first = threadIdx.x * per * 4;
+  int32_t mine = 0;
+  for (int i = 0; i < per; ++i) {
+    const int4 v = mine4[i];
+    const int k = first + 4 * i;
+    mine += (k < total ? v.x : 0) + (k + 1 < total ? v.y : 0) + (k + 2 < total ? v.z : 0) + (k + 3 < total ? v.w : 0);
+  }
+  int32_t incl = mine;
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) {
+    const int32_t v = __shfl_up(incl, s, 64);
+    if (l >= s) incl += v;
+  }
+  if (l == 63) wave_total[w] = incl;
+  __syncthreads();
+  int32_t base = incl - mine;
+  for (int k = 0; k < w; ++k) base += wave_total[k];
+  for (int i = 0; i < per; ++i) {   // past `total` only padding is written
+    const int4 v = mine4[i];
+    int4 o;
+    o.x = base;
+    o.y = o.x + v.x;
+    o.z = o.y + v.y;
+    o.w = o.z + v.z;
+    base = o.w + v.w;
+    mine4[i] = o;
+  }
+  if (!ptr) return;
+  __syncthreads();
+  if ((int)threadIdx.x < digits) ptr[threadIdx.x] = counts[threadIdx.x * tiles];
+  if (threadIdx.x == 0) ptr[digits] = (int32_t)E;
+}
+
+__global__ __launch_bounds__(256) void sort_scatter_kernel(const int64_t* __restrict__ keys,
+                                                           const int32_t* __restrict__ k32,
+                                                           const int32_t* __restrict__ ids, int64_t E, int64_t N,
+                                                           int shift, int digits, const int32_t* __restrict__ base,
+                                                           int32_t* __restrict__ k_out, int32_t* __restrict__ ids_out) {
+  __shared__ int32_t hist[kSortWaves][kDigits];
+  int32_t key[kRounds], rank[kRounds];
+  tile_histogram(keys, k32, E, N, shift, hist, key, rank);
+  {   // this digit's base of each wave: the tile's scanned base plus the earlier waves' counts
+    const int d = threadIdx.x;
+    int32_t t = d < digits ? base[(int64_t)d * gridDim.x + blockIdx.x] : 0;
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) {
+      const int32_t v = hist[w][d];
+      hist[w][d] = t;
+      t += v;
+    }
+  }
+  __syncthreads();
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+#pragma unroll
+  for (int r = 0; r < kRounds; ++r) {
+    const int64_t i = (int64_t)blockIdx.x * kTile + w * (kTile / kSortWaves) + r * 64 + l;
+    if (i >= E) continue;
+    const int32_t at = hist[w][(key[r] >> shift) & (kDigits - 1)] + rank[r];
+    if (k_out) k_out[at] = key[r];
+    ids_out[at] = ids ? ids[i] : (int32_t)i;
+  }
+}
+
+// Bytes of a pass's counts: whole groups of four for every thread of the scan.
+size_t count_bytes(int64_t tiles) { return sizeof(int32_t) * 4096 * (size_t)((kDigits * tiles + 4095) / 4096); }
+
+// Passes of the counting sort, or 0 where the library sort is used: more than 2^16 keys would need a third
+// pass, and the one-block scan of [256][tiles] grows with the list.
+constexpr int64_t kSmallSort = int64_t(1) << 18;
+int sort_passes(int64_t E, int64_t N) {
+  if (E > kSmallSort || N >= (int64_t(1) << 16)) return 0;
+  return N < kDigits ? 1 : 2;
+}
+
 // ---- Spatial (Morton) row order -------------------------------------------
 // Spread the low 10 bits of v so that bit i moves to bit 3i.
 __device__ __forceinline__ uint32_t spread3(uint32_t v) {
@@ -367,6 +520,10 @@ int ictc_tp_bwd(int li, int le, int lo, int C, const float* x, const float* sh, 
 
 int64_t ictc_csr_workspace_bytes(int64_t E, int64_t N) {
   if (E < 0 || N < 0 || E >= (int64_t(1) << 31) || N >= (int64_t(1) << 31) - 2) return -1;
+  if (sort_passes(E, N)) {
+    const size_t tiles = (size_t)(E > 0 ? (E + kTile - 1) / kTile : 1);
+    return (int64_t)(count_bytes((int64_t)tiles) + align256(3 * sizeof(int32_t) * (size_t)(E > 0 ? E : 1)));
+  }
   return (int64_t)(3 * align256(sizeof(int32_t) * (size_t)(E > 0 ? E : 1)) + align256(sort_temp_bytes(E, N)));
 }
 
@@ -393,6 +550,30 @@ int ictc_csr_build(const int64_t* keys, int64_t E, int64_t N, int32_t* ptr, int3
     return fail(ICTC_ERR_ARGUMENT, "csr: workspace of %lld bytes, need %lld", (long long)workspace_bytes,
                 (long long)need);
   char* ws = (char*)workspace;
+  if (const int passes = sort_passes(E, N)) {
+    const int64_t tiles = (E + kTile - 1) / kTile;
+    int32_t* counts = (int32_t*)ws;
+    int32_t* k1 = (int32_t*)(ws + count_bytes(tiles));
+    int32_t* id1 = k1 + E;
+    int32_t* k2 = id1 + E;
+    const dim3 grid((unsigned)tiles), block(256);
+    const bool two = passes == 2;
+    const int d0 = two ? kDigits : (int)N + 1, d1 = (int)(N >> 8) + 1;
+    hipLaunchKernelGGL(sort_count_kernel, grid, block, 0, st, keys, (const int32_t*)nullptr, E, N, 0, d0, counts);
+    hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(1024), 0, st, counts, d0, (int)tiles, E,
+                       two ? nullptr : ptr);
+    hipLaunchKernelGGL(sort_scatter_kernel, grid, block, 0, st, keys, (const int32_t*)nullptr, (const int32_t*)nullptr,
+                       E, N, 0, d0, counts, two ? k1 : nullptr, two ? id1 : order);
+    if (two) {
+      hipLaunchKernelGGL(sort_count_kernel, grid, block, 0, st, keys, k1, E, N, 8, d1, counts);
+      hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(1024), 0, st, counts, d1, (int)tiles, E,
+                         (int32_t*)nullptr);
+      hipLaunchKernelGGL(sort_scatter_kernel, grid, block, 0, st, keys, k1, id1, E, N, 8, d1, counts, k2,
+                         order);
+      hipLaunchKernelGGL(csr_ptr_kernel, dim3((unsigned)((N + 2 + 255) / 256)), dim3(256), 0, st, k2, E, N, ptr);
+    }
+    return check_hip(hipGetLastError(), "csr counting sort");
+  }
   const size_t slab = align256(sizeof(int32_t) * (size_t)E);
   int32_t* k_in = (int32_t*)ws;
   int32_t* k_out = (int32_t*)(ws + slab);

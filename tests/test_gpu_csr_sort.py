@@ -1,0 +1,22 @@
+"""The CSR of unsorted keys (ictc_csr_build) is exactly the stable sort by key, on both sides of every rule."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("E,N", [(1, 1), (63, 3), (1024, 255), (1025, 254), (4097, 10), (5000, 256), (70001, 1359),
+                                 (20000, 65535), (3000, 65536), (262144, 4096), (262145, 4096)])
+def test_csr_is_a_stable_sort(device, E, N):
+    """Both digit passes, tile and stretch edges, ids out of range (last), and the library sort's side of the rule."""
+    from ictc_o3.ops.tensor_product import Csr
+    g = torch.Generator().manual_seed(E)
+    keys = torch.randint(0, N, (E,), generator=g)
+    if E > 10:
+        keys[::7] = N - 1                     # a long segment
+        keys[3], keys[5] = -2, N + 9
+    k = torch.where((keys < 0) | (keys >= N), torch.full_like(keys, N), keys)
+    csr = Csr(keys.to(device), N)
+    assert torch.equal(csr.order[:E].long().cpu(), torch.argsort(k, stable=True))
+    want = torch.cat([torch.searchsorted(k.sort().values, torch.arange(N + 1)), torch.tensor([E])])
+    assert torch.equal(csr.ptr.long().cpu(), want)
