@@ -158,7 +158,7 @@ size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 // digit's scanned base for the tile, plus the counts of the tile's earlier waves, plus that of the wave's
 // earlier keys (ballots of equal digits), so equal digits keep their order.  Up to 255 distinct keys (species
 // ids) one pass sorts and its scan yields ptr; receiver lists of up to 65,535 rows take two.  Measured (us of
-// kernels): 65,000 edges over 1,359 receivers 65 -> 44 and 10 launches -> 7; 8,191 species ids 37 -> 14 and
+// kernels): 65,000 edges over 1,359 receivers 65 -> 40 and 10 launches -> 7; 8,191 species ids 37 -> 15 and
 // 8 -> 3.
 constexpr int kDigits = 256, kTile = 1024, kSortWaves = 4, kRounds = kTile / (64 * kSortWaves);
 

@@ -5,6 +5,7 @@
 
 #include "../../include/ictc_mi355x.h"
 #include "sc_launch.h"
+#include "sc_table.h"
 
 namespace ictc {
 // Shared with capi.hip (error reporting).
@@ -68,6 +69,23 @@ struct GetShape {
   int run() {
     *out = shape_of<T>();
     return ICTC_OK;
+  }
+};
+
+// Dispatch onto the shapes with a coefficient-table form; `none` for the others.
+template <class F>
+int dispatch_tab(int li, int lt, int corr, int none, F&& f) {
+#define ICTC_SC_CASE(A, B, C) \
+  if (li == A && lt == B && corr == C) return f.template run<ictc::Sc<A, B, C>, ictc::ScTab<A, B, C>>();
+  ICTC_FOR_EACH_SC_TAB(ICTC_SC_CASE)
+#undef ICTC_SC_CASE
+  return none;
+}
+
+struct TabPairs {
+  template <class T, class Tab>
+  int run() {
+    return Tab::PAIRS;
   }
 };
 
@@ -137,9 +155,119 @@ struct Dw {
   }
 };
 
+// Table build, then out (mode 0..3 of tab_kernel).
+struct TabApply {
+  ictc::sc::TabArgs a;
+  ictc::ScWeights w;
+  float* table;
+  const float *go, *h;
+  float* out;
+  int mode;
+  hipStream_t st;
+  template <class T, class Tab>
+  int run() {
+    using L = ictc::sc::TabLaunch<T>;
+    if (int rc = hip_status(L::table(w, a.num_species, a.channels, table, st), "sc coefficient table launch")) return rc;
+    return hip_status(L::apply(a, go, h, out, mode, st), "sc table launch");
+  }
+};
+
+struct TabDw {
+  ictc::sc::TabArgs a;
+  const float *go, *h;
+  float* const* dw;
+  float* partial;
+  hipStream_t st;
+  template <class T, class Tab>
+  int run() {
+    return hip_status(ictc::sc::TabLaunch<T>::dw(a, go, h, dw, partial, st), "sc table dw launch");
+  }
+};
+
+ictc::sc::TabArgs tab_args(const float* x, const float* table, const int32_t* ptr, const int32_t* order, int64_t N,
+                           int S, int C) {
+  ictc::sc::TabArgs a;
+  a.x = x;
+  a.table = table;
+  a.ptr = ptr;
+  a.order = order;
+  a.nodes = N;
+  a.num_species = S;
+  a.channels = C;
+  return a;
+}
+
+// Common checks of the table entry points; *floats = workspace floats of the coefficient table (dw = 0) or of
+// the pair sums (dw = 1).
+int check_tab(int li, int lt, int corr, int C, int S, int64_t N, int dw, Shape* sh, int64_t* floats) {
+  if (int rc = check_common(li, lt, corr, C, S, N, sh)) return rc;
+  const int64_t pairs = dispatch_tab(li, lt, corr, 0, TabPairs{});
+  if (pairs == 0)
+    return fail(ICTC_ERR_UNSUPPORTED, "symmetric contraction (lmax=%d, target_lmax=%d, correlation=%d) has no table form",
+                li, lt, corr);
+  if (S > 65535) return fail(ICTC_ERR_UNSUPPORTED, "symmetric contraction table: more than 65535 species");
+  if (N >= (int64_t(1) << 31)) return fail(ICTC_ERR_UNSUPPORTED, "symmetric contraction table: more than 2^31 nodes");
+  *floats = dw ? (ictc::sc::tab_max_chunks(N, pairs, C, S) + S) * pairs * C : ictc::sc::tab_floats(pairs, C, S);
+  return ICTC_OK;
+}
+
 }  // namespace
 
 extern "C" {
+
+int ictc_sc_table_pairs(int lmax, int target_lmax, int correlation) {
+  return dispatch_tab(lmax, target_lmax, correlation, 0, TabPairs{});
+}
+
+int64_t ictc_sc_table_workspace_bytes(int lmax, int target_lmax, int correlation, int channels, int64_t nodes,
+                                      int num_species, int weight_gradients) {
+  Shape sh;
+  int64_t floats;
+  if (check_tab(lmax, target_lmax, correlation, channels, num_species, nodes, weight_gradients, &sh, &floats)) return -1;
+  return floats * (int64_t)sizeof(float);
+}
+
+// Derivatives: grad selects the feature gradient, tangent the derivative of either along it.
+int ictc_sc_table_apply(int li, int lt, int corr, int C, const float* x, int S, const float* const* weights, int64_t N,
+                        const int32_t* species_ptr, const int32_t* species_order, const float* grad,
+                        const float* tangent, float* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  Shape sh;
+  int64_t floats;
+  if (int rc = check_tab(li, lt, corr, C, S, N, 0, &sh, &floats)) return rc;
+  if (N == 0) return ICTC_OK;
+  if (!x || !species_ptr || !species_order || !out || !workspace)
+    return fail(ICTC_ERR_ARGUMENT, "ictc_sc_table_apply: null operand");
+  if (int rc = check_weights(weights, sh)) return rc;
+  if (workspace_bytes < floats * (int64_t)sizeof(float))
+    return fail(ICTC_ERR_ARGUMENT, "ictc_sc_table_apply: workspace of %lld bytes, need %lld", (long long)workspace_bytes,
+                (long long)(floats * (int64_t)sizeof(float)));
+  float* table = (float*)workspace;
+  const Args w = make_args(x, nullptr, weights, N, S, C, sh);
+  return dispatch_tab(li, lt, corr, ICTC_ERR_UNSUPPORTED,
+                      TabApply{tab_args(x, table, species_ptr, species_order, N, S, C), w.w, table, grad, tangent, out,
+                               (grad ? 2 : 0) + (tangent ? 1 : 0), (hipStream_t)stream});
+}
+
+int ictc_sc_table_bwd_w(int li, int lt, int corr, int C, const float* x, int S, int64_t N, const float* grad,
+                        const float* tangent, const int32_t* species_ptr, const int32_t* species_order,
+                        float* const* dweights, void* workspace, int64_t workspace_bytes, void* stream) {
+  Shape sh;
+  int64_t floats;
+  if (int rc = check_tab(li, lt, corr, C, S, N, 1, &sh, &floats)) return rc;
+  if (!dweights) return fail(ICTC_ERR_ARGUMENT, "null weight-gradient table");
+  for (int L = 0; L < 4; ++L)
+    for (int n = 0; n < 3; ++n)
+      if (sh.P[L][n] > 0 && !dweights[L * 3 + n])
+        return fail(ICTC_ERR_ARGUMENT, "null weight gradient for L=%d nu=%d", L, n + 1);
+  if ((N > 0 && (!x || !grad || !species_order)) || !species_ptr || !workspace)
+    return fail(ICTC_ERR_ARGUMENT, "ictc_sc_table_bwd_w: null operand");
+  if (workspace_bytes < floats * (int64_t)sizeof(float))
+    return fail(ICTC_ERR_ARGUMENT, "ictc_sc_table_bwd_w: workspace of %lld bytes, need %lld", (long long)workspace_bytes,
+                (long long)(floats * (int64_t)sizeof(float)));
+  return dispatch_tab(li, lt, corr, ICTC_ERR_UNSUPPORTED,
+                      TabDw{tab_args(x, nullptr, species_ptr, species_order, N, S, C), grad, tangent, dweights,
+                            (float*)workspace, (hipStream_t)stream});
+}
 
 int ictc_sc_shape(int lmax, int target_lmax, int correlation, int* paths, int* num_weights) {
   Shape sh;

@@ -106,6 +106,10 @@ _SIGNATURES = {
     "ictc_sc_terms": (_i, [_i, _i, _i]),
     "ictc_sc_shape": (_i, [_i, _i, _i, _p, _p]),
     "ictc_sc_workspace_bytes": (_i64, [_i, _i, _i, _i, _i64, _i]),
+    "ictc_sc_table_pairs": (_i, [_i, _i, _i]),
+    "ictc_sc_table_workspace_bytes": (_i64, [_i, _i, _i, _i, _i64, _i, _i]),
+    "ictc_sc_table_apply": (_i, [_i, _i, _i, _i, _p, _i, _p, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
+    "ictc_sc_table_bwd_w": (_i, [_i, _i, _i, _i, _p, _i, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "ictc_sc_fwd": (_i, [_i, _i, _i, _i, _p, _p, _i, _p, _i64, _p, _p]),
     "ictc_sc_bwd_x": (_i, [_i, _i, _i, _i, _p, _p, _i, _p, _i64, _p, _p, _p]),
     "ictc_sc_bwd_w": (_i, [_i, _i, _i, _i, _p, _i, _i64, _p, _p, _p, _p, _p, _i64, _p]),

@@ -42,6 +42,8 @@ class ScSpec:
         self.paths, self.num_weights = sc_shape(lmax, target_lmax, correlation)
         self.nx = (lmax + 1) ** 2
         self.no = sum(2 * L + 1 for L in range(target_lmax + 1))
+        # (output, monomial) pairs of the table kernels, 0 where the shape has none
+        self.pairs = int(nat.lib().ictc_sc_table_pairs(lmax, target_lmax, correlation))
         # flattened (L, nu) slots that carry weights, in table order
         self.slots = [(L, n) for L in range(target_lmax + 1) for n in range(correlation) if self.paths[L][n] > 0]
 
@@ -72,7 +74,39 @@ def term_count(spec) -> int:
     return n
 
 
-def _fwd_raw(spec, x, species, ws, tangent=None):
+# The table kernels form each pair's weight combination once per species and evaluate three or four nodes of a
+# species per wave; they need the species-sorted node order and the table.  Below these many (node, 64-channel
+# group) waves the per-node kernels are as fast (one wave per node fills more of the GPU): lmax 3 over 2,048
+# nodes of 64 channels 54 -> 36 us forward but 17 us for the order; lmax 2, whose terms outnumber its pairs less,
+# 18 -> 19 us over 8,000 nodes and 266 -> 190 over 131,072 (its weight gradients, which take the order anyway,
+# 85 -> 68 and 1,390 -> 515).  With few nodes per species the table costs what it saves.
+_TABLE_WAVES = {3: 4096, 2: 32768}
+_TABLE_WEIGHT_WAVES = 4096
+_TABLE_NODES_PER_SPECIES = 32
+
+
+def _use_table(spec, N, weights=False) -> bool:
+    waves = N * ((spec.channels + 63) // 64)
+    return (spec.pairs > 0 and waves >= (_TABLE_WEIGHT_WAVES if weights else _TABLE_WAVES[spec.lmax])
+            and N >= _TABLE_NODES_PER_SPECIES * spec.num_species)
+
+
+def _table_raw(spec, x, csr, ws, go=None, tangent=None):
+    """SC(x), its tangent, or with go the feature gradient or its tangent, on the coefficient tables."""
+    N = x.shape[0]
+    out = x.new_empty(N, spec.no * spec.channels) if go is None else torch.empty_like(x)
+    nbytes = int(nat.lib().ictc_sc_table_workspace_bytes(spec.lmax, spec.target_lmax, spec.corr, spec.channels, N,
+                                                         spec.num_species, 0))
+    work = x.new_empty(max(nbytes, 4) // 4)
+    nat.call("ictc_sc_table_apply", spec.lmax, spec.target_lmax, spec.corr, spec.channels, nat.ptr(x),
+             spec.num_species, _table(spec, ws), N, nat.ptr(csr.ptr), nat.ptr(csr.order), nat.ptr(go),
+             nat.ptr(tangent), nat.ptr(out), nat.ptr(work), nbytes, nat.stream_of(x))
+    return out
+
+
+def _fwd_raw(spec, x, species, ws, tangent=None, holder=None):
+    if holder is not None and _use_table(spec, x.shape[0]):
+        return _table_raw(spec, x, holder.species_csr().csr, ws, tangent=tangent)
     out = x.new_empty(x.shape[0], spec.no * spec.channels)
     if tangent is None:
         nat.call("ictc_sc_fwd", spec.lmax, spec.target_lmax, spec.corr, spec.channels, nat.ptr(x), nat.ptr(species),
@@ -83,7 +117,9 @@ def _fwd_raw(spec, x, species, ws, tangent=None):
     return out
 
 
-def _dx_raw(spec, x, species, ws, go, tangent=None):
+def _dx_raw(spec, x, species, ws, go, tangent=None, holder=None):
+    if holder is not None and _use_table(spec, x.shape[0]):
+        return _table_raw(spec, x, holder.species_csr().csr, ws, go, tangent)
     dx = torch.empty_like(x)
     if tangent is None:
         nat.call("ictc_sc_bwd_x", spec.lmax, spec.target_lmax, spec.corr, spec.channels, nat.ptr(x),
@@ -99,6 +135,15 @@ def _dx_raw(spec, x, species, ws, go, tangent=None):
 def _dw_raw(spec, x, species_csr, go, tangent=None):
     N = x.shape[0]
     dws = [x.new_empty(spec.num_species, spec.paths[L][n], spec.channels) for L, n in spec.slots]
+    if _use_table(spec, N, weights=True):
+        nbytes = int(nat.lib().ictc_sc_table_workspace_bytes(spec.lmax, spec.target_lmax, spec.corr, spec.channels, N,
+                                                             spec.num_species, 1))
+        work = x.new_empty(max(nbytes, 4) // 4)
+        csr = species_csr.csr
+        nat.call("ictc_sc_table_bwd_w", spec.lmax, spec.target_lmax, spec.corr, spec.channels, nat.ptr(x),
+                 spec.num_species, N, nat.ptr(go), nat.ptr(tangent), nat.ptr(csr.ptr), nat.ptr(csr.order),
+                 _table(spec, dws), nat.ptr(work), nbytes, nat.stream_of(x))
+        return dws
     ws_bytes = int(nat.lib().ictc_sc_workspace_bytes(spec.lmax, spec.target_lmax, spec.corr, spec.channels, N,
                                                      spec.num_species))
     work = x.new_empty(max(ws_bytes // 4, 1))
@@ -125,7 +170,7 @@ class _SC(torch.autograd.Function):
         x = _c(x)
         ws = tuple(_c(w) for w in ws)
         ctx.save_for_backward(x, *ws)
-        return _fwd_raw(spec, x, species, ws)
+        return _fwd_raw(spec, x, species, ws, holder=holder)
 
     @staticmethod
     def backward(ctx, go):
@@ -145,7 +190,7 @@ class _SCAdjoint(torch.autograd.Function):
         ctx.set_materialize_grads(False)
         ctx.spec, ctx.species, ctx.holder = spec, species, holder
         ctx.save_for_backward(x, go, *ws)
-        dx = _dx_raw(spec, x, species, ws, go) if need_x else None
+        dx = _dx_raw(spec, x, species, ws, go, holder=holder) if need_x else None
         dws = _dw_raw(spec, x, holder.species_csr(), go) if need_w else [None] * len(ws)
         return (dx, *dws)
 
@@ -163,15 +208,15 @@ class _SCAdjoint(torch.autograd.Function):
         dws = [None] * len(ws)
         if n_go:
             if hdx is not None:
-                dgo = _fwd_raw(spec, x, species, ws, tangent=_c(hdx))
+                dgo = _fwd_raw(spec, x, species, ws, tangent=_c(hdx), holder=holder)
             if have_hw:
-                t = _fwd_raw(spec, x, species, hws)
+                t = _fwd_raw(spec, x, species, hws, holder=holder)
                 dgo = t if dgo is None else dgo + t
         if n_x:
             if hdx is not None:
-                dx = _dx_raw(spec, x, species, ws, go, tangent=_c(hdx))
+                dx = _dx_raw(spec, x, species, ws, go, tangent=_c(hdx), holder=holder)
             if have_hw:
-                t = _dx_raw(spec, x, species, hws, go)
+                t = _dx_raw(spec, x, species, hws, go, holder=holder)
                 dx = t if dx is None else dx + t
         if any(n_w) and hdx is not None:
             dws = _dw_raw(spec, x, holder.species_csr(), go, tangent=_c(hdx))
@@ -179,20 +224,25 @@ class _SCAdjoint(torch.autograd.Function):
 
 
 class _SpeciesHolder:
-    """Lazily built species-sorted node CSR, shared by the adjoints of one forward call."""
+    """Lazily built species-sorted node CSR, shared by the adjoints of one forward call (shared=True: the
+    model's order of this step's species tensor, which its self connections use as well)."""
 
-    def __init__(self, species, num_species):
-        self.species, self.num_species, self._csr = species, num_species, None
+    def __init__(self, species, num_species, shared=False):
+        self.species, self.num_species, self.shared, self._csr = species, num_species, shared, None
 
     def species_csr(self):
         if self._csr is None:
-            self._csr = _SpeciesCsr(self.species, self.num_species)
+            if self.shared:
+                from ictc_o3.ops.linear import species_order
+                self._csr = species_order(self.species, self.num_species)
+            else:
+                self._csr = _SpeciesCsr(self.species, self.num_species)
         return self._csr
 
 
-def symmetric_contraction(x, species, weights: List[torch.Tensor], spec: ScSpec):
+def symmetric_contraction(x, species, weights: List[torch.Tensor], spec: ScSpec, shared_order=False):
     """x [N, NX*C] packed ir_mul, species [N] int64, weights in spec.slots order -> [N, NO*C] packed ir_mul."""
-    holder = _SpeciesHolder(species, spec.num_species)
+    holder = _SpeciesHolder(species, spec.num_species, shared_order)
     return _SC.apply(spec, species, holder, x, *weights)
 
 
@@ -259,9 +309,9 @@ class ICTDBridgeUSymmetricContractionSO3(nn.Module):
         spec = self.spec()
         return [self.symmetric_contractions.contractions[L].weight_for(n + 1) for L, n in spec.slots]
 
-    def contract(self, x, species):
+    def contract(self, x, species, shared_order=False):
         """Native entry: x [N, (lmax+1)^2*C] packed ir_mul -> [N, sum_L (2L+1)*C] packed ir_mul."""
-        return symmetric_contraction(x, species, self.slot_weights(), self.spec())
+        return symmetric_contraction(x, species, self.slot_weights(), self.spec(), shared_order)
 
     def forward(self, node_feats, node_attrs=None, node_type_idx=None):
         """Reference layout: flat mul_ir in and out (symmetric_contraction.py:98-147)."""

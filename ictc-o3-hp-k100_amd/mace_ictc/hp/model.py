@@ -214,7 +214,7 @@ class Product(nn.Module):
         self.linear = ProductLinear(channels, target_lmax)
 
     def forward(self, message, sc, species, first_order=False):
-        out = self.linear(self.symmetric_contractions.contract(message, species), first_order)
+        out = self.linear(self.symmetric_contractions.contract(message, species, shared_order=True), first_order)
         C = self.channels
         if out.shape[1] == C:
             return out + sc

@@ -682,6 +682,30 @@ int ictc_sc_bwd_w_jvp(int lmax, int target_lmax, int correlation, int channels, 
                       const int32_t* species_order, float* const* dweights, void* workspace,
                       int64_t workspace_bytes, void* stream);
 
+/* The same maps for many nodes, over per-species coefficient tables: the weight
+ * combination of every (output, monomial) pair is formed once per species instead
+ * of once per node, and nodes are taken in species order (species_ptr /
+ * species_order from ictc_csr_build(species, nodes, num_species); nodes past
+ * species_ptr[num_species] have an id out of range and get zero rows).  Correlation
+ * 3 with (lmax, target_lmax) in {(2,2), (3,1), (3,2)}: ictc_sc_table_pairs
+ * gives the pair count, 0 for the other shapes.
+ *   apply: out = SC(x), with tangent its J_x h; with grad the feature gradient,
+ *          with grad and tangent Hess_x(grad . out) h;
+ *   bwd_w: dW as ictc_sc_bwd_w, with tangent as ictc_sc_bwd_w_jvp.
+ * workspace: ictc_sc_table_workspace_bytes(..., weight_gradients = 0 for apply, 1
+ * for bwd_w) bytes (-1: no table form or an argument out of range).            */
+int ictc_sc_table_pairs(int lmax, int target_lmax, int correlation);
+int64_t ictc_sc_table_workspace_bytes(int lmax, int target_lmax, int correlation, int channels, int64_t nodes,
+                                      int num_species, int weight_gradients);
+int ictc_sc_table_apply(int lmax, int target_lmax, int correlation, int channels, const float* x, int num_species,
+                        const float* const* weights, int64_t nodes, const int32_t* species_ptr,
+                        const int32_t* species_order, const float* grad, const float* tangent, float* out,
+                        void* workspace, int64_t workspace_bytes, void* stream);
+int ictc_sc_table_bwd_w(int lmax, int target_lmax, int correlation, int channels, const float* x, int num_species,
+                        int64_t nodes, const float* grad, const float* tangent, const int32_t* species_ptr,
+                        const int32_t* species_order, float* const* dweights, void* workspace,
+                        int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
