@@ -416,13 +416,6 @@ __global__ void fill_zero_i32_kernel(int32_t* __restrict__ p, int64_t n) {
   if (i < n) p[i] = 0;
 }
 
-hipError_t route_edge_fwd(const ictc::TpShape& s, const ictc::Operands& a, float* out, hipStream_t st) {
-  return ictc::launch_edge_fwd(s, a, out, st);
-}
-hipError_t route_edge_bwd(const ictc::TpShape& s, const ictc::Operands& a, const float* grad, float* dx, float* dsh,
-                          float* dg, float* ws, hipStream_t st) {
-  return ictc::launch_edge_bwd(s, a, grad, dx, dsh, dg, ws, st);
-}
 hipError_t route_msg_fwd(const ictc::TpShape& s, const ictc::Operands& a, const int64_t* src, ictc::Csr c,
                          float* out, hipStream_t st) {
   return ictc::launch_msg_fwd(s, a, src, c, out, st);
@@ -488,15 +481,25 @@ int ictc_tp_shape(int input_lmax, int edge_lmax, int output_lmax, int* num_paths
   return ICTC_OK;
 }
 
-int ictc_tp_fwd(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
-                int64_t E, float* out, void* stream) {
+static int tp_fwd(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
+                  int64_t E, float* out, bool mul_ir, void* stream) {
   if (int rc = check_shape(li, le, lo, C)) return rc;
   if (E < 0) return fail(ICTC_ERR_ARGUMENT, "edges must be nonnegative");
   if (E == 0) return ICTC_OK;
   if (!x || !sh || !g || !out) return fail(ICTC_ERR_ARGUMENT, "ictc_tp_fwd: null operand");
   const ictc::TpShape s{li, le, lo, C};
-  return check_hip(route_edge_fwd(s, operands(x, sh, g, w, nullptr, E, E, C), out, (hipStream_t)stream),
+  return check_hip(ictc::launch_edge_fwd(s, operands(x, sh, g, w, nullptr, E, E, C), out, mul_ir, (hipStream_t)stream),
                    "ictc_tp_fwd launch");
+}
+
+int ictc_tp_fwd(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
+                int64_t E, float* out, void* stream) {
+  return tp_fwd(li, le, lo, C, x, sh, g, w, E, out, false, stream);
+}
+
+int ictc_tp_fwd_mul_ir(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
+                       int64_t E, float* out, void* stream) {
+  return tp_fwd(li, le, lo, C, x, sh, g, w, E, out, true, stream);
 }
 
 int64_t ictc_tp_workspace_bytes(int edge_lmax, int channels, int64_t edges) {
@@ -504,18 +507,30 @@ int64_t ictc_tp_workspace_bytes(int edge_lmax, int channels, int64_t edges) {
   return group_ws_floats(edge_lmax, channels, edges) * (int64_t)sizeof(float);
 }
 
-int ictc_tp_bwd(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
-                const float* grad, int64_t E, float* dx, float* dsh, float* dg, void* workspace,
-                int64_t workspace_bytes, void* stream) {
+static int tp_bwd(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
+                  const float* grad, int64_t E, float* dx, float* dsh, float* dg, void* workspace,
+                  int64_t workspace_bytes, bool mul_ir, void* stream) {
   if (int rc = check_shape(li, le, lo, C)) return rc;
   if (E < 0) return fail(ICTC_ERR_ARGUMENT, "edges must be nonnegative");
   if (E == 0 || (!dx && !dsh && !dg)) return ICTC_OK;
   if (!x || !sh || !g || !grad) return fail(ICTC_ERR_ARGUMENT, "ictc_tp_bwd: null operand");
   if (int rc = check_ws(dsh, (const float*)workspace, workspace_bytes, le, C, E, "ictc_tp_bwd")) return rc;
   const ictc::TpShape s{li, le, lo, C};
-  return check_hip(route_edge_bwd(s, operands(x, sh, g, w, nullptr, E, E, C), grad, dx, dsh, dg, (float*)workspace,
-                                         (hipStream_t)stream),
+  return check_hip(ictc::launch_edge_bwd(s, operands(x, sh, g, w, nullptr, E, E, C), grad, dx, dsh, dg,
+                                         (float*)workspace, mul_ir, (hipStream_t)stream),
                    "ictc_tp_bwd launch");
+}
+
+int ictc_tp_bwd(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
+                const float* grad, int64_t E, float* dx, float* dsh, float* dg, void* workspace,
+                int64_t workspace_bytes, void* stream) {
+  return tp_bwd(li, le, lo, C, x, sh, g, w, grad, E, dx, dsh, dg, workspace, workspace_bytes, false, stream);
+}
+
+int ictc_tp_bwd_mul_ir(int li, int le, int lo, int C, const float* x, const float* sh, const float* g, const float* w,
+                       const float* grad, int64_t E, float* dx, float* dsh, float* dg, void* workspace,
+                       int64_t workspace_bytes, void* stream) {
+  return tp_bwd(li, le, lo, C, x, sh, g, w, grad, E, dx, dsh, dg, workspace, workspace_bytes, true, stream);
 }
 
 int64_t ictc_csr_workspace_bytes(int64_t E, int64_t N) {

@@ -17,9 +17,9 @@ struct TpShape {
 // Channel groups of 64 for a channel count (0: unsupported).
 inline int channel_groups(int C) { return C < 1 || C > 64 * kMaxGroups ? 0 : (C + 63) / 64; }
 
-hipError_t launch_edge_fwd(const TpShape& s, const Operands& a, float* out, hipStream_t st);
+hipError_t launch_edge_fwd(const TpShape& s, const Operands& a, float* out, bool mul_ir, hipStream_t st);
 hipError_t launch_edge_bwd(const TpShape& s, const Operands& a, const float* grad, float* dx, float* dsh, float* dg,
-                           float* ws, hipStream_t st);
+                           float* ws, bool mul_ir, hipStream_t st);
 hipError_t launch_msg_fwd(const TpShape& s, const Operands& a, const int64_t* src, Csr dcsr, float* out,
                           hipStream_t st);
 // The source-owned feature adjoint gathers a 9 KB receiver cotangent row per

@@ -26,6 +26,8 @@ _SIGNATURES = {
     "ictc_last_error": (ctypes.c_char_p, []),
     "ictc_tp_shape": (_i, [_i, _i, _i, ctypes.POINTER(_i), ctypes.POINTER(_i)]),
     "ictc_tp_fwd": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _i64, _p, _p]),
+    "ictc_tp_fwd_mul_ir": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _i64, _p, _p]),
+    "ictc_tp_bwd_mul_ir": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _i64, _p]),
     "ictc_tp_workspace_bytes": (_i64, [_i, _i, _i64]),
     "ictc_tp_bwd": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _i64, _p]),
     "ictc_tp_second": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _i64, _p]),

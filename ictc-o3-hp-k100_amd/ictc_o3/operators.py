@@ -170,24 +170,6 @@ class EdgeTensorProduct(torch.nn.Module):
             offset += count * self.tp.channels * width
         return result
 
-    def _features_to_ir_mul(self, features):
-        C, parts, off = self.tp.channels, [], 0
-        for l in range(self.input_lmax + 1):
-            w = C * (2 * l + 1)
-            parts.append(features[:, off:off + w].reshape(-1, C, 2 * l + 1).transpose(1, 2).reshape(-1, w))
-            off += w
-        return torch.cat(parts, -1)
-
-    def _output_to_mul_ir(self, output):
-        C, parts, off = self.tp.channels, [], 0
-        for l in range(self.tp.lmax + 1):
-            count, width = self.tp.path_counts_by_l.get(l, 0), 2 * l + 1
-            w = count * C * width
-            if w:
-                parts.append(output[:, off:off + w].reshape(-1, count, width, C).transpose(2, 3).reshape(-1, w))
-            off += w
-        return torch.cat(parts, -1)
-
     def forward(self, features, harmonics, gates):
         """features [E,C*(L_in+1)^2], harmonics [E,(L_edge+1)^2], gates [E,P*C] or [E,P,C] (operators.py:310-340)."""
         _tp_coverage(self.tp, self.input_lmax, self.edge_lmax)
@@ -203,12 +185,7 @@ class EdgeTensorProduct(torch.nn.Module):
             empty = features[:, :1] * harmonics[:, :1] * gates.reshape(0, self.gate_width)[:, :1]
             return empty.expand(0, self.output_width)
         spec = self._prepare()
-        if self.layout == "mul_ir":
-            features = self._features_to_ir_mul(features)
-        out = tpo.edge_tp(features, harmonics, gates.reshape(rows, self.gate_width), spec)
-        if self.layout == "mul_ir":
-            out = self._output_to_mul_ir(out)
-        return out
+        return tpo.edge_tp(features, harmonics, gates.reshape(rows, self.gate_width), spec, self.layout == "mul_ir")
 
 
 def _index_vector(value, e, device, name, message):

@@ -77,10 +77,10 @@ def _add(a, b):
 # ---------------------------------------------------------------------------
 
 
-def _edge_fwd_raw(spec, x, sh, g):
+def _edge_fwd_raw(spec, x, sh, g, mul_ir=False):
     E = x.shape[0]
     out = x.new_empty(E, spec.out_components * spec.channels)
-    nat.call("ictc_tp_fwd", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh), nat.ptr(g),
+    nat.call("ictc_tp_fwd_mul_ir" if mul_ir else "ictc_tp_fwd", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh), nat.ptr(g),
              _w(spec), E, nat.ptr(out), nat.stream_of(x))
     return out
 
@@ -95,13 +95,13 @@ def _group_ws(spec, E, dsh):
     return torch.empty(nbytes // 4, dtype=torch.float32, device=dsh.device), nbytes
 
 
-def _edge_bwd_raw(spec, x, sh, g, go, need):
+def _edge_bwd_raw(spec, x, sh, g, go, need, mul_ir=False):
     E = x.shape[0]
     dx = torch.empty_like(x) if need[0] else None
     dsh = torch.empty_like(sh) if need[1] else None
     dg = torch.empty_like(g) if need[2] else None
     ws, ws_bytes = _group_ws(spec, E, dsh)
-    nat.call("ictc_tp_bwd", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh), nat.ptr(g),
+    nat.call("ictc_tp_bwd_mul_ir" if mul_ir else "ictc_tp_bwd", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh), nat.ptr(g),
              _w(spec), nat.ptr(go), E, nat.ptr(dx), nat.ptr(dsh), nat.ptr(dg), nat.ptr(ws), ws_bytes,
              nat.stream_of(x))
     return dx, dsh, dg
@@ -118,8 +118,32 @@ def _second_outputs(need, tx, tsh, tg):
             ng and (tx is not None or tsh is not None), ngo and any(t is not None for t in (tx, tsh, tg)))
 
 
-def _edge_second_raw(spec, x, sh, g, go, tx, tsh, tg, need):
-    """Fused mixed second derivative of the edge TP adjoint (one kernel); returns (dx, dsh, dg, dgo)."""
+def _turn_rows(t, widths, channels, to_ir_mul):
+    """Rows [E, sum(widths) * C] between [channel, magnetic] and [magnetic, channel] order within each block."""
+    if t is None:
+        return None
+    out = torch.empty_like(t)
+    off = 0
+    for w in widths:
+        n = w * channels
+        shape, turned = ((channels, w), (w, channels)) if to_ir_mul else ((w, channels), (channels, w))
+        out[:, off:off + n].unflatten(1, turned).copy_(t[:, off:off + n].unflatten(1, shape).transpose(1, 2))
+        off += n
+    return out
+
+
+def _edge_second_raw(spec, x, sh, g, go, tx, tsh, tg, need, mul_ir=False):
+    """Fused mixed second derivative of the edge TP adjoint (one kernel); returns (dx, dsh, dg, dgo).
+    mul_ir rows are rewritten for the kernel and back."""
+    if mul_ir:
+        from ictc_o3.basis import tables
+        C = spec.channels
+        ins = [2 * l + 1 for l in range(spec.li + 1)]
+        paths = tables.natural_paths(spec.li, spec.le, spec.lo)
+        outs = [2 * l + 1 for l in range(spec.lo + 1) for p in paths if p[2] == l]
+        turned = [_turn_rows(_c(t) if t is not None else None, w, C, True) for t, w in ((x, ins), (go, outs), (tx, ins))]
+        dx, dsh, dg, dgo = _edge_second_raw(spec, turned[0], sh, g, turned[1], turned[2], tsh, tg, need)
+        return _turn_rows(dx, ins, C, False), dsh, dg, _turn_rows(dgo, outs, C, False)
     E = x.shape[0]
     tx, tsh, tg = _tangents(tx, tsh, tg)
     wx, wsh, wg, wgo = _second_outputs(need, tx, tsh, tg)
@@ -137,76 +161,77 @@ def _edge_second_raw(spec, x, sh, g, go, tx, tsh, tg, need):
 
 class EdgeTP(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, sh, g, spec):
+    def forward(ctx, x, sh, g, spec, mul_ir=False):
         ctx.set_materialize_grads(False)
-        ctx.spec = spec
+        ctx.spec, ctx.mul_ir = spec, mul_ir
         x, sh, g = _c(x), _c(sh), _c(g)
         ctx.save_for_backward(x, sh, g)
-        return _edge_fwd_raw(spec, x, sh, g)
+        return _edge_fwd_raw(spec, x, sh, g, mul_ir)
 
     @staticmethod
     def backward(ctx, go):
         if go is None:
-            return None, None, None, None
+            return None, None, None, None, None
         x, sh, g = ctx.saved_tensors
         need = required_gradients((x, sh, g), ctx.needs_input_grad[:3])
         if not any(need):
-            return None, None, None, None
-        dx, dsh, dg = EdgeTPAdjoint.apply(x, sh, g, _c(go), ctx.spec, need)
-        return dx, dsh, dg, None
+            return None, None, None, None, None
+        dx, dsh, dg = EdgeTPAdjoint.apply(x, sh, g, _c(go), ctx.spec, need, ctx.mul_ir)
+        return dx, dsh, dg, None, None
 
 
-def edge_tp(x, sh, g, spec):
-    return EdgeTP.apply(x, sh, g, spec)
+def edge_tp(x, sh, g, spec, mul_ir=False):
+    """Per-edge TP; mul_ir: x, the output and their gradients are [channel, magnetic] rows."""
+    return EdgeTP.apply(x, sh, g, spec, mul_ir)
 
 
-def edge_adjoint(x, sh, g, go, spec, need):
-    return EdgeTPAdjoint.apply(x, sh, g, go, spec, need)
+def edge_adjoint(x, sh, g, go, spec, need, mul_ir=False):
+    return EdgeTPAdjoint.apply(x, sh, g, go, spec, need, mul_ir)
 
 
 class EdgeTPAdjoint(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, sh, g, go, spec, need):
+    def forward(ctx, x, sh, g, go, spec, need, mul_ir=False):
         ctx.set_materialize_grads(False)
-        ctx.spec = spec
+        ctx.spec, ctx.mul_ir = spec, mul_ir
         x, sh, g, go = _c(x), _c(sh), _c(g), _c(go)
         ctx.save_for_backward(x, sh, g, go)
-        return _edge_bwd_raw(spec, x, sh, g, go, need)
+        return _edge_bwd_raw(spec, x, sh, g, go, need, mul_ir)
 
     @staticmethod
     def backward(ctx, hx, hsh, hg):
         x, sh, g, go = ctx.saved_tensors
-        spec = ctx.spec
+        spec, mul_ir = ctx.spec, ctx.mul_ir
         nx, nsh, ng, ngo = required_gradients((x, sh, g, go), ctx.needs_input_grad[:4])
         if not torch.is_grad_enabled():
             # the mixed second derivative itself is the last order asked for: one fused kernel
-            dx, dsh, dg, dgo = _edge_second_raw(spec, x, sh, g, go, hx, hsh, hg, (nx, nsh, ng, ngo))
-            return dx, dsh, dg, dgo, None, None
+            dx, dsh, dg, dgo = _edge_second_raw(spec, x, sh, g, go, hx, hsh, hg, (nx, nsh, ng, ngo), mul_ir)
+            return dx, dsh, dg, dgo, None, None, None
         # higher orders: compose differentiable first-order operators (multilinearity)
         dx = dsh = dg = dgo = None
         if ngo:
             if hx is not None:
-                dgo = _add(dgo, edge_tp(hx, sh, g, spec))
+                dgo = _add(dgo, edge_tp(hx, sh, g, spec, mul_ir))
             if hsh is not None:
-                dgo = _add(dgo, edge_tp(x, hsh, g, spec))
+                dgo = _add(dgo, edge_tp(x, hsh, g, spec, mul_ir))
             if hg is not None:
-                dgo = _add(dgo, edge_tp(x, sh, hg, spec))
+                dgo = _add(dgo, edge_tp(x, sh, hg, spec, mul_ir))
         if nx:
             if hsh is not None:
-                dx = _add(dx, edge_adjoint(x, hsh, g, go, spec, (True, False, False))[0])
+                dx = _add(dx, edge_adjoint(x, hsh, g, go, spec, (True, False, False), mul_ir)[0])
             if hg is not None:
-                dx = _add(dx, edge_adjoint(x, sh, hg, go, spec, (True, False, False))[0])
+                dx = _add(dx, edge_adjoint(x, sh, hg, go, spec, (True, False, False), mul_ir)[0])
         if nsh:
             if hx is not None:
-                dsh = _add(dsh, edge_adjoint(hx, sh, g, go, spec, (False, True, False))[1])
+                dsh = _add(dsh, edge_adjoint(hx, sh, g, go, spec, (False, True, False), mul_ir)[1])
             if hg is not None:
-                dsh = _add(dsh, edge_adjoint(x, sh, hg, go, spec, (False, True, False))[1])
+                dsh = _add(dsh, edge_adjoint(x, sh, hg, go, spec, (False, True, False), mul_ir)[1])
         if ng:
             if hx is not None:
-                dg = _add(dg, edge_adjoint(hx, sh, g, go, spec, (False, False, True))[2])
+                dg = _add(dg, edge_adjoint(hx, sh, g, go, spec, (False, False, True), mul_ir)[2])
             if hsh is not None:
-                dg = _add(dg, edge_adjoint(x, hsh, g, go, spec, (False, False, True))[2])
-        return dx, dsh, dg, dgo, None, None
+                dg = _add(dg, edge_adjoint(x, hsh, g, go, spec, (False, False, True), mul_ir)[2])
+        return dx, dsh, dg, dgo, None, None, None
 
 
 # ---------------------------------------------------------------------------

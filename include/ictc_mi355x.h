@@ -66,6 +66,19 @@ int ictc_tp_bwd(int input_lmax, int edge_lmax, int output_lmax, int channels,
                 float* dfeatures, float* dharmonics, float* dgates, void* workspace,
                 int64_t workspace_bytes, void* stream);
 
+/* ictc_tp_fwd / ictc_tp_bwd on rows in the reference's "mul_ir" layout
+ * (operators.py:283-308): within each degree (features) or path slot (out, grad)
+ * block of 2l+1 components the order is [channel, magnetic] instead of
+ * [magnetic, channel].  Gates and harmonics as above.                         */
+int ictc_tp_fwd_mul_ir(int input_lmax, int edge_lmax, int output_lmax, int channels,
+                       const float* features, const float* harmonics, const float* gates,
+                       const float* weight, int64_t edges, float* out, void* stream);
+int ictc_tp_bwd_mul_ir(int input_lmax, int edge_lmax, int output_lmax, int channels,
+                       const float* features, const float* harmonics, const float* gates,
+                       const float* weight, const float* grad, int64_t edges,
+                       float* dfeatures, float* dharmonics, float* dgates, void* workspace,
+                       int64_t workspace_bytes, void* stream);
+
 /* Mixed second derivative of ictc_tp_bwd: the derivative of the first
  * adjoint (features, harmonics, gates; grad) -> (dfeatures, dharmonics,
  * dgates) along tangents tfeatures / tharmonics / tgates of its three outputs
