@@ -137,6 +137,63 @@ def tp_struct(li, le, lo):
                          f" t = fmaf(y[{j}], b, t); }}")
         lines.append(f"      d[{p}] = fmaf(go[{k}], t, d[{p}]); }}{SB}")
     lines.append("  }")
+    # dy and the tangent dot of one x, path by path: as dydg, with dgt += gt[p] dg[p] taken as each path ends, so
+    # no dg array lives through the body.  The fence after each path hides that x is unchanged: without it the
+    # products C x_i common to several paths stay in registers (over 100 for the degree-3 triples).
+    by_pk = {}
+    for p, i, j, k, v in ent:
+        by_pk.setdefault(p, {}).setdefault(k, {}).setdefault(j, []).append((i, v))
+    lines.append("  __device__ __forceinline__ static void dydgt(float* __restrict__ x, const float* __restrict__ y,"
+                 " const float* __restrict__ gw, const float* __restrict__ gt, const float* __restrict__ go,"
+                 " float* __restrict__ dyv, float& dgt) {")
+    for p in range(P):
+        lines.append("    { float u = 0.f;")
+        for k, js in sorted(by_pk.get(p, {}).items()):
+            lines.append(f"      {{ const float w = gw[{p}] * go[{k}]; float t = 0.f;")
+            for j, terms in sorted(js.items()):
+                lines.append(f"        {{ const float b = {b_expr('x', terms)}; dyv[{j}] = fmaf(w, b, dyv[{j}]);"
+                             f" t = fmaf(y[{j}], b, t); }}")
+            lines.append(f"        u = fmaf(go[{k}], t, u); }}")
+        used = sorted({i for js in by_pk.get(p, {}).values() for terms in js.values() for i, _ in terms})
+        lines.append(f"      dgt = fmaf(gt[{p}], u, dgt); }}")
+        lines.append("    " + " ".join(f'asm volatile("" : "+v"(x[{i}]));' for i in used))
+    lines.append("  }")
+    def fence(p):
+        used = sorted({i for js in by_pk.get(p, {}).values() for terms in js.values() for i, _ in terms})
+        return "    " + " ".join(f'asm volatile("" : "+v"(x[{i}]));' for i in used)
+
+    # the three forward terms of the mixed second derivative together, path by path:
+    #   o[k] += gw[p] sum_j (y[j] B_jk(tx) + ty[j] B_jk(x)) + tg[p] sum_j y[j] B_jk(x)
+    # (B_jk(x) formed once for both of its terms)
+    lines.append("  __device__ __forceinline__ static void fwd3_f(float* __restrict__ x, float* __restrict__ tx,"
+                 " const float* __restrict__ y, const float* __restrict__ ty, const float* __restrict__ gw,"
+                 " const float* __restrict__ tg, float* __restrict__ o) {")
+    for p in range(P):
+        for k, js in sorted(by_pk.get(p, {}).items()):
+            lines.append("    { float s = 0.f, t = 0.f;")
+            for j, terms in sorted(js.items()):
+                lines.append(f"      {{ const float b = {b_expr('x', terms)}; s = fmaf(ty[{j}], b, s); t = fmaf(y[{j}], b, t); }}")
+                lines.append(f"      {{ const float b = {b_expr('tx', terms)}; s = fmaf(y[{j}], b, s); }}")
+            lines.append(f"      o[{k}] = fmaf(tg[{p}], t, fmaf(gw[{p}], s, o[{k}])); }}")
+        lines.append(fence(p))
+        lines.append(fence(p).replace("(x[", "(tx["))
+    lines.append("  }")
+    # the two feature-gradient terms of the mixed second derivative together, V_p formed once for both:
+    #   d[i] += gw[p] sum_j V_p[i][j] ty[j] + tg[p] sum_j V_p[i][j] y[j]
+    by_pij2 = {}
+    for p, i, j, k, v in ent:
+        by_pij2.setdefault(p, {}).setdefault(i, {}).setdefault(j, []).append((k, v))
+    lines.append("  __device__ __forceinline__ static void dx2_v(const float* __restrict__ y, const float* __restrict__ ty,"
+                 " const float* __restrict__ gw, const float* __restrict__ tg, const float* __restrict__ go,"
+                 " float* __restrict__ d) {")
+    for p in range(P):
+        for i, js in sorted(by_pij2.get(p, {}).items()):
+            lines.append("    { float s = 0.f, t = 0.f;")
+            for j, ks in sorted(js.items()):
+                lines.append(f"      {{ const float v = {' + '.join(f'{f(v)} * go[{k}]' for k, v in ks)};"
+                             f" s = fmaf(v, ty[{j}], s); t = fmaf(v, y[{j}], t); }}")
+            lines.append(f"      d[{i}] = fmaf(tg[{p}], t, fmaf(gw[{p}], s, d[{i}])); }}")
+    lines.append("  }")
     # dx, dy and dg together, factorised through V_p[i][j] = sum_{k in p} C go[k] (one op per nonzero):
     #   d[i]   += gw[p] sum_j V_p[i][j] y[j]
     #   dyv[j] += gw[p] sum_i V_p[i][j] x[i]

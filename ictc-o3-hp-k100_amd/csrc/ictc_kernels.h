@@ -732,19 +732,21 @@ __device__ __forceinline__ float gate_tangent_dot(const Operands& a, const float
 // Receiver-owned adjoint: per-edge gate and harmonic gradients.  Waves of
 // row `rows` own the out-of-range tail segment ptr[rows]..ptr[rows+1] and
 // write zero gradients for it (mask 0, zero cotangent).
-// Waves per SIMD of the receiver-owned adjoint: the gate-tangent form holds the
-// tangent row besides the gate row and the full dy/dg contraction, so it asks
-// for one wave per SIMD fewer than the table (at the table's level up to 113
-// VGPRs spill, e.g. Tp<2,3,3>; one fewer leaves at most 5).
+// Waves per SIMD of the receiver-owned adjoint.  The gate-tangent form takes the table's count but at least 2: its
+// path-by-path contraction (Tp::dydgt) holds no gate-gradient array and no products shared between paths, and
+// with the harmonic gradient chosen at launch it compiles without spills at 2 waves up to (2,3,3) (202 VGPRs; the
+// slot-ordered form with a run-time choice took 316, one wave per SIMD, and its loads' latency showed: (2,3,3)
+// C128 over 206 k edges 1,321 -> 828 us) and with 5 spilled VGPRs at (3,3,3).
 template <class T, bool TAN>
 constexpr int edge_adjoint_waves() {
   constexpr int w = Occupancy<kMsgBwdEdge, T::LI, T::LE, T::LO>::value;
-  return (TAN && w > 1) ? w - 1 : w;
+  return TAN && w < 2 ? 2 : w;
 }
 
 // With TAN, gdot [E, P*C] (d gates / dr) replaces the gate gradient output:
 // dr[e] = sum dgates * gdot is written instead (group g > 0: slab g-1 of dr_part).
-template <class T, bool TAN>
+// DSH: the harmonic gradient is written too (chosen at launch); without TAN it is tested at run time.
+template <class T, bool TAN, bool DSH = false>
 __global__ __launch_bounds__(kBlock, (edge_adjoint_waves<T, TAN>())) void msg_bwd_edge_kernel(
     Operands a, const int64_t* __restrict__ src, Csr csr, const float* __restrict__ grad, float* __restrict__ dsh,
     float* __restrict__ dsh_part, float* __restrict__ dgates, int parts, const float* __restrict__ gdot,
@@ -787,12 +789,20 @@ __global__ __launch_bounds__(kBlock, (edge_adjoint_waves<T, TAN>())) void msg_bw
         load_row<T::NX>(a.x + s * (int64_t)(T::NX * C), C, c, xv);
         load_gw<T>(a, lane_i(ch.row, i), c, m, gw);
         load_row<T::P>(gdot + lane_i(ch.row, i) * (int64_t)(T::P * C), C, c, gt);
-        if (dsh) T::dydg(xv, y, gw, go, dyv, d);
-        else T::dg(xv, y, go, d);
-        dgt = m * gate_tangent_dot<T>(a, gdot, e, c, gt, d);
+        if constexpr (DSH) {
+          if (a.weight) {
+#pragma unroll
+            for (int p = 0; p < T::P; ++p) gt[p] *= a.weight[p * C + c];
+          }
+          T::dydgt(xv, y, gw, gt, go, dyv, dgt);
+          dgt *= m;
+        } else {
+          T::dg(xv, y, go, d);
+          dgt = m * gate_tangent_dot<T>(a, gdot, e, c, gt, d);
+        }
       }
       if (TAN) {
-        store_dsh_dr<T::NY>(dsh_g, dr_g, e, dyv, dgt);
+        store_dsh_dr<T::NY>(DSH ? dsh_g : nullptr, dr_g, e, dyv, dgt);
         continue;
       }
       if (active) {

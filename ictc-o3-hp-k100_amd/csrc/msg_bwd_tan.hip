@@ -29,8 +29,12 @@ struct MsgBwdTan {
       if ((err = hipGetLastError()) != hipSuccess) return err;
     } else {
       const int parts = row_parts(a.rows + 1, G);
-      hipLaunchKernelGGL((msg_bwd_edge_kernel<T, true>), dim3(blocks_for((a.rows + 1) * parts), G), dim3(kBlock), 0,
-                         st, a, src, dcsr, grad, dsh, ws, nullptr, parts, gdot, dr, ws_dr);
+      if (dsh)
+        hipLaunchKernelGGL((msg_bwd_edge_kernel<T, true, true>), dim3(blocks_for((a.rows + 1) * parts), G),
+                           dim3(kBlock), 0, st, a, src, dcsr, grad, dsh, ws, nullptr, parts, gdot, dr, ws_dr);
+      else
+        hipLaunchKernelGGL((msg_bwd_edge_kernel<T, true, false>), dim3(blocks_for((a.rows + 1) * parts), G),
+                           dim3(kBlock), 0, st, a, src, dcsr, grad, dsh, ws, nullptr, parts, gdot, dr, ws_dr);
       if ((err = hipGetLastError()) != hipSuccess) return err;
       if (dx) {
         hipLaunchKernelGGL((msg_bwd_x_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock),

@@ -18,8 +18,12 @@ struct MsgSecondRcv {
     const int G = channel_groups(a.channels);
     if (dgrad) {
       const int sum = sum_parts(a.rows, G, kSumWaves);
-      hipLaunchKernelGGL((msg_fwd2_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t, src, csr,
-                         dgrad, sum);
+      if (t.x && t.sh && t.gates)
+        hipLaunchKernelGGL((msg_fwd2_kernel<T, true>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t, src,
+                           csr, dgrad, sum);
+      else
+        hipLaunchKernelGGL((msg_fwd2_kernel<T, false>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t,
+                           src, csr, dgrad, sum);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
     }

@@ -15,8 +15,12 @@ struct MsgSecondSrc {
   template <class T>
   hipError_t run() {
     const int G = channel_groups(a.channels), sum = sum_parts(a.rows, G, kSourceSumWaves);
-    hipLaunchKernelGGL((msg_bwd_x2_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t, dst, csr,
-                       grad, dx, sum);
+    if (t.sh && t.gates)
+      hipLaunchKernelGGL((msg_bwd_x2_kernel<T, true>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t, dst,
+                         csr, grad, dx, sum);
+    else
+      hipLaunchKernelGGL((msg_bwd_x2_kernel<T, false>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock), 0, st, a, t,
+                         dst, csr, grad, dx, sum);
     return hipGetLastError();
   }
 };
