@@ -152,7 +152,7 @@ def exported_symbols():
 
 
 def call(name: str, *args) -> None:
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
         msg = lib().ictc_last_error().decode(errors="replace")
         if rc in (-1, -2):
@@ -161,13 +161,13 @@ def call(name: str, *args) -> None:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()   # c_void_p parameters take integers
 
 
 def stream_of(t: torch.Tensor):
     if t.device.type != "cuda":
         raise ValueError("ICTC MI355X kernels require tensors on a ROCm (cuda) device")
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def tp_shape(li: int, le: int, lo: int):

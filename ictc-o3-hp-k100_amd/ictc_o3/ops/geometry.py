@@ -74,16 +74,8 @@ class _EdgeHarmonics(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, pos, shift, topo, cutoff, lmax, uses):
-        pos = _c(pos.detach())
-        shift = None if shift is None else _c(shift.detach())
-        E, N = topo.src.numel(), pos.shape[0]
-        r = pos.new_empty(E)
-        n = pos.new_empty(E, 3)
-        mask = pos.new_empty(E)
-        Y = pos.new_empty(E, (lmax + 1) ** 2)
-        nat.call("ictc_edge_harmonics_fwd", nat.ptr(pos), nat.ptr(shift), nat.ptr(topo.src), nat.ptr(topo.dst), N,
-                 E, float(cutoff), lmax, nat.ptr(r), nat.ptr(n), nat.ptr(mask), nat.ptr(Y), nat.stream_of(pos))
-        ctx.topo, ctx.nodes, ctx.lmax, ctx.uses = topo, N, lmax, uses
+        r, n, mask, Y = edge_harmonics_raw(pos, shift, topo, cutoff, lmax)
+        ctx.topo, ctx.nodes, ctx.lmax, ctx.uses = topo, pos.shape[0], lmax, uses
         ctx.mark_non_differentiable(mask)
         ctx.save_for_backward(r, n)
         if uses == 2:
@@ -98,15 +90,33 @@ class _EdgeHarmonics(torch.autograd.Function):
         else:
             (dr, dY, _dmask), dr2, dY2 = grads, None, None
         r, n = ctx.saved_tensors
-        E = r.numel()
-        dvec = r.new_empty(E, 3)
-        cot = [None if g is None else _c(g) for g in (dr, dY, dr2, dY2)]
-        # the kernel reads dY / dY2 as 16-byte vectors
-        cot = [g if g is None or k in (0, 2) or g.data_ptr() % 16 == 0 else g.clone() for k, g in enumerate(cot)]
-        nat.call("ictc_edge_harmonics_bwd", nat.ptr(r), nat.ptr(n), *[nat.ptr(g) for g in cot], E, ctx.lmax,
-                 nat.ptr(dvec), nat.stream_of(r))
+        dvec = edge_harmonics_adjoint_raw(r, n, (dr, dY, dr2, dY2), ctx.lmax)
         dpos = _vector_adjoint(dvec, ctx.topo, ctx.nodes) if ctx.needs_input_grad[0] else None
         return dpos, (dvec if ctx.needs_input_grad[1] else None), None, None, None, None
+
+
+def edge_harmonics_raw(pos, shift, topo, cutoff: float, lmax: int):
+    """(r, n, mask, Y) of the edges (no autograd)."""
+    pos = _c(pos.detach())
+    shift = None if shift is None else _c(shift.detach())
+    E, N = topo.src.numel(), pos.shape[0]
+    r, n, mask = pos.new_empty(E), pos.new_empty(E, 3), pos.new_empty(E)
+    Y = pos.new_empty(E, (lmax + 1) ** 2)
+    nat.call("ictc_edge_harmonics_fwd", nat.ptr(pos), nat.ptr(shift), nat.ptr(topo.src), nat.ptr(topo.dst), N,
+             E, float(cutoff), lmax, nat.ptr(r), nat.ptr(n), nat.ptr(mask), nat.ptr(Y), nat.stream_of(pos))
+    return r, n, mask, Y
+
+
+def edge_harmonics_adjoint_raw(r, n, cotangents, lmax: int):
+    """d vec [E, 3] for the cotangents (dr, dY, dr', dY'), each or None, of edge_harmonics (no autograd)."""
+    E = r.numel()
+    dvec = r.new_empty(E, 3)
+    cot = [None if g is None else _c(g) for g in cotangents]
+    # the kernel reads dY / dY2 as 16-byte vectors
+    cot = [g if g is None or k in (0, 2) or g.data_ptr() % 16 == 0 else g.clone() for k, g in enumerate(cot)]
+    nat.call("ictc_edge_harmonics_bwd", nat.ptr(r), nat.ptr(n), *[nat.ptr(g) for g in cot], E, lmax,
+             nat.ptr(dvec), nat.stream_of(r))
+    return dvec
 
 
 def edge_harmonics(pos: torch.Tensor, shift: torch.Tensor | None, topo, cutoff: float, lmax: int, uses: int = 1):

@@ -283,14 +283,12 @@ class _PackedLinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, layout, *weights):
-        lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
         ctx.layout = layout
         ctx.inputs = (x, *weights)
         x = x if x.is_contiguous() else x.contiguous()
         ws = [_weight_operand(w) for w in weights]
         ctx.save_for_backward(x, *ws)
-        return _packed_call(x, Ci, Co, lmax, pin, in_off, [1] * (lmax + 1), out_off, ws, scales,
-                            (lmax + 1) ** 2 * Co)
+        return packed_linear_raw(x, layout, ws)
 
     @staticmethod
     def backward(ctx, dout):
@@ -308,10 +306,7 @@ def _packed_adjoint(x, ws, layout, dout, needs):
     """Input adjoint (needs[0]) and weight gradients (needs[1:]) of the packed linear for cotangent dout."""
     lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
     dout = dout if dout.is_contiguous() else dout.contiguous()
-    dx = None
-    if needs[0]:
-        wt = [_weight_operand(w, transpose=True) for w in ws]
-        dx = _packed_call(dout, Co, Ci, lmax, [1] * (lmax + 1), out_off, pin, in_off, wt, scales, in_cols)
+    dx = packed_linear_adjoint_raw(dout, layout, ws) if needs[0] else None
     dws = []
     N = x.shape[0]
     for l, (w, need) in enumerate(zip(ws, needs[1:])):
@@ -339,14 +334,12 @@ class _LayerEntry(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, h, layout, C, *weights):
-        lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
         ctx.layout, ctx.C = layout, C
         ctx.inputs = (h, *weights)
         x = h if h.is_contiguous() else h.contiguous()
         ws = [_weight_operand(w) for w in weights]
         ctx.save_for_backward(x, *ws)
-        y = _packed_call(x, Ci, Co, lmax, pin, in_off, [1] * (lmax + 1), out_off, ws, scales, (lmax + 1) ** 2 * Co)
-        return y, x[:, :C].contiguous()
+        return packed_linear_raw(x, layout, ws), x[:, :C].contiguous()
 
     @staticmethod
     def backward(ctx, dy, ds):
@@ -368,10 +361,7 @@ def layer_entry_fast(h, weights, C, lmax):
     """(degree_linear(h), h[:, :C]) on the MFMA kernel with a fused input adjoint (first derivatives only)."""
     if not _fast_ok(h, weights, C) or h.shape[1] == C:
         return None
-    Co = weights[0].shape[0]
-    layout = (lmax, C, Co, [1] * (lmax + 1), [l * l * C for l in range(lmax + 1)],
-              [l * l * Co for l in range(lmax + 1)], [1.0] * (lmax + 1), (lmax + 1) ** 2 * C)
-    return _LayerEntry.apply(h, layout, C, *weights[:lmax + 1])
+    return _LayerEntry.apply(h, degree_layout(weights, C, lmax), C, *weights[:lmax + 1])
 
 
 class _AddScalars(torch.autograd.Function):
@@ -562,21 +552,43 @@ def degree_linear_fast(x, weights, C, lmax, scale=1.0):
     """degree_linear on the MFMA kernel (first derivatives only)."""
     if not _fast_ok(x, weights, C):
         return degree_linear(x, weights, C, lmax, scale)
-    Co = weights[0].shape[0]
-    layout = (lmax, C, Co, [1] * (lmax + 1), [l * l * C for l in range(lmax + 1)],
-              [l * l * Co for l in range(lmax + 1)], [float(scale)] * (lmax + 1), (lmax + 1) ** 2 * C)
-    return _PackedLinear.apply(x, layout, *weights[:lmax + 1])
+    return _PackedLinear.apply(x, degree_layout(weights, C, lmax, scale), *weights[:lmax + 1])
 
 
 def path_linear_fast(m, weights, counts, C, lmax, scale=1.0):
     """path_linear on the MFMA kernel (first derivatives only)."""
     if not _fast_ok(m, weights, C) or any(counts.get(l, 0) == 0 for l in range(lmax + 1)):
         return path_linear(m, weights, counts, C, lmax, scale)
+    return _PackedLinear.apply(m, path_layout(weights, counts, C, lmax, scale), *weights[:lmax + 1])
+
+
+def degree_layout(weights, C, lmax, scale=1.0):
+    """_PackedLinear layout of the degree-wise channel map."""
+    Co = weights[0].shape[0]
+    return (lmax, C, Co, [1] * (lmax + 1), [l * l * C for l in range(lmax + 1)],
+            [l * l * Co for l in range(lmax + 1)], [float(scale)] * (lmax + 1), (lmax + 1) ** 2 * C)
+
+
+def path_layout(weights, counts, C, lmax, scale=1.0):
+    """_PackedLinear layout of the map from the path slots of each degree."""
     Co = weights[0].shape[0]
     pin, in_off, off = [], [], 0
     for l in range(lmax + 1):
         pin.append(counts[l])
         in_off.append(off)
         off += counts[l] * (2 * l + 1) * C
-    layout = (lmax, C, Co, pin, in_off, [l * l * Co for l in range(lmax + 1)], [float(scale)] * (lmax + 1), off)
-    return _PackedLinear.apply(m, layout, *weights[:lmax + 1])
+    return (lmax, C, Co, pin, in_off, [l * l * Co for l in range(lmax + 1)], [float(scale)] * (lmax + 1), off)
+
+
+def packed_linear_raw(x, layout, weights):
+    """The packed linear of a _PackedLinear layout (no autograd)."""
+    lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
+    return _packed_call(x, Ci, Co, lmax, pin, in_off, [1] * (lmax + 1), out_off, [_weight_operand(w) for w in weights],
+                        scales, (lmax + 1) ** 2 * Co)
+
+
+def packed_linear_adjoint_raw(dout, layout, weights):
+    """Its input adjoint."""
+    lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
+    wt = [_weight_operand(w, transpose=True) for w in weights]
+    return _packed_call(dout, Co, Ci, lmax, [1] * (lmax + 1), out_off, pin, in_off, wt, scales, in_cols)

@@ -123,6 +123,24 @@ class _WeightGrad(torch.autograd.Function):
         return da, db
 
 
+def edge_linear_raw(x, W):
+    """x W^T (no autograd)."""
+    if x.is_cuda and x.shape[0] >= _TN_MIN_ROWS and x.shape[1] == 64 and W.shape[0] % 16 == 0:
+        return gate_projection(x, W)   # split-bf16 MFMA, FP32-level accuracy (hidden layers and projection)
+    if _own_gemm(x):
+        return gemm_nt(x, W)
+    return x @ W.t()
+
+
+def edge_linear_adjoint_raw(u, W):
+    """u W (no autograd)."""
+    if u.is_cuda and u.shape[0] >= _TN_MIN_ROWS and W.shape[1] == 64 and W.shape[0] % 64 == 0:
+        return gate_projection_adjoint(u, W)   # split-bf16 MFMA, FP32-level accuracy
+    if _own_gemm(u):
+        return gemm_nt(u, W.t())
+    return u @ W
+
+
 class _EdgeLinear(torch.autograd.Function):
     """y = x W^T over edge rows; the weight gradient runs on the split-reduction kernel."""
 
@@ -130,11 +148,7 @@ class _EdgeLinear(torch.autograd.Function):
     def forward(ctx, x, W):
         ctx.save_for_backward(x, W)
         ctx.inputs = (x, W)
-        if x.is_cuda and x.shape[0] >= _TN_MIN_ROWS and x.shape[1] == 64 and W.shape[0] % 16 == 0:
-            return gate_projection(x, W)   # split-bf16 MFMA, FP32-level accuracy (hidden layers and projection)
-        if _own_gemm(x):
-            return gemm_nt(x, W)
-        return x @ W.t()
+        return edge_linear_raw(x, W)
 
     @staticmethod
     def backward(ctx, g):
@@ -154,12 +168,7 @@ class _EdgeLinearT(torch.autograd.Function):
     def forward(ctx, u, W):
         ctx.save_for_backward(u, W)
         ctx.inputs = (u, W)
-        M = W.shape[0]
-        if u.is_cuda and u.shape[0] >= _TN_MIN_ROWS and W.shape[1] == 64 and M % 64 == 0:
-            return gate_projection_adjoint(u, W)   # split-bf16 MFMA, FP32-level accuracy
-        if _own_gemm(u):
-            return gemm_nt(u, W.t())
-        return u @ W
+        return edge_linear_adjoint_raw(u, W)
 
     @staticmethod
     def backward(ctx, h):

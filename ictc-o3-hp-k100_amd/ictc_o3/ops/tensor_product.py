@@ -773,10 +773,16 @@ SPECIES_FORM = True
 SPECIES_MAX = 4
 
 
+def species_form(spec, num_species: int) -> bool:
+    """Whether the shape runs in the species form."""
+    return (SPECIES_FORM and spec.li == 0 and spec.le == spec.lo and spec.le <= 2
+            and 1 <= num_species <= SPECIES_MAX)
+
+
 def _species_ok(spec, x, xtab):
-    return (SPECIES_FORM and xtab is not None and spec.li == 0 and spec.le == spec.lo and spec.le <= 2
+    return (xtab is not None and species_form(spec, xtab.shape[0])
             and x.is_cuda and x.dtype == torch.float32 and xtab.dtype == torch.float32
-            and 1 <= xtab.shape[0] <= SPECIES_MAX and xtab.shape[1] == spec.channels)
+            and xtab.shape[1] == spec.channels)
 
 
 class SpeciesRadialMessage(torch.autograd.Function):
@@ -803,21 +809,9 @@ class SpeciesRadialMessage(torch.autograd.Function):
         x, sh, rc = _c(x), _c(sh), _c(r.detach())
         Ws = [_c(w.detach()) for w in (W1, W2, W3, W4)]
         xtab, species = _c(xtab.detach()), _c(species)
-        E, N, S = rc.shape[0], x.shape[0], xtab.shape[0]
-        rg = _c(topo.gate_input(rc))
+        h3, t3 = _mlp_tangent_raw(topo.gate_input(rc), Ws, cfg)
         ctx.rows = topo.gate_rows
-        h3, t3 = rc.new_empty(rg.shape[0], 64), rc.new_empty(rg.shape[0], 64)
-        nat.call("ictc_radial_mlp_tangent_fwd", nat.ptr(rg), rg.shape[0], 8, 64, float(cfg[0]), int(cfg[1]),
-                 nat.ptr(Ws[0]), nat.ptr(Ws[1]), nat.ptr(Ws[2]), float(cfg[2]), nat.ptr(h3), nat.ptr(t3),
-                 nat.stream_of(rc))
-        out = x.new_empty(N, spec.out_components * spec.channels)
-        ws, nbytes = _species_ws(spec, S, N, x.device)
-        tok = _timing.begin(f"species_fwd[{spec.le}C{spec.channels}S{S}]")
-        nat.call("ictc_species_message_fwd", spec.le, spec.lo, spec.channels, S, nat.ptr(xtab), nat.ptr(species),
-                 nat.ptr(sh), nat.ptr(h3), nat.ptr(Ws[3]), _w(spec), nat.ptr(mask), nat.ptr(topo.src), N, E,
-                 nat.ptr(topo.by_dst.ptr), nat.ptr(topo.by_dst.order), nat.ptr(topo.dst_rows), nat.ptr(ctx.rows),
-                 nat.ptr(out), nat.ptr(ws), nbytes, nat.stream_of(x))
-        _timing.end(tok)
+        out = _species_fwd_raw(spec, topo, xtab, species, sh, h3, Ws[3], mask, ctx.rows)
         ctx.save_for_backward(x, sh, rc, *Ws, h3, t3, xtab, species)
         return out
 
@@ -840,16 +834,69 @@ class SpeciesRadialMessage(torch.autograd.Function):
             return (dx, dsh, dr, *dW, *rest)
         if not (needs[1] or needs[2]):
             return (None,) * 13
-        N, E, S = x.shape[0], sh.shape[0], xtab.shape[0]
-        dsh, dr = torch.empty_like(sh), sh.new_empty(E)
-        ws, nbytes = _species_ws(spec, S, N, x.device)
-        tok = _timing.begin(f"species_bwd[{spec.le}C{spec.channels}S{S}]")
-        nat.call("ictc_species_message_bwd", spec.le, spec.lo, spec.channels, S, nat.ptr(xtab), nat.ptr(species),
-                 nat.ptr(sh), nat.ptr(h3), nat.ptr(t3), nat.ptr(W4), _w(spec), nat.ptr(mask), nat.ptr(topo.src),
-                 N, E, nat.ptr(topo.by_dst.ptr), nat.ptr(topo.by_dst.order), nat.ptr(topo.dst_rows),
-                 nat.ptr(ctx.rows), nat.ptr(go), nat.ptr(dsh), nat.ptr(dr), nat.ptr(ws), nbytes, nat.stream_of(x))
-        _timing.end(tok)
+        dsh, dr = _species_bwd_raw(spec, topo, xtab, species, sh, h3, t3, W4, mask, go, ctx.rows)
         return (None, dsh if needs[1] else None, dr if needs[2] else None, None, None, None, None, *rest)
+
+
+def _mlp_tangent_raw(r, Ws, cfg):
+    """Last hidden activation of the radial MLP and its r tangent, [rows, 64] each, for lengths r."""
+    r = _c(r)
+    h3, t3 = r.new_empty(r.shape[0], 64), r.new_empty(r.shape[0], 64)
+    nat.call("ictc_radial_mlp_tangent_fwd", nat.ptr(r), r.shape[0], 8, 64, float(cfg[0]), int(cfg[1]),
+             nat.ptr(Ws[0]), nat.ptr(Ws[1]), nat.ptr(Ws[2]), float(cfg[2]), nat.ptr(h3), nat.ptr(t3), nat.stream_of(r))
+    return h3, t3
+
+
+def _species_fwd_raw(spec, topo, xtab, species, sh, h3, W4, mask, rows):
+    N, E, S = species.shape[0], sh.shape[0], xtab.shape[0]
+    out = sh.new_empty(N, spec.out_components * spec.channels)
+    ws, nbytes = _species_ws(spec, S, N, sh.device)
+    tok = _timing.begin(f"species_fwd[{spec.le}C{spec.channels}S{S}]")
+    nat.call("ictc_species_message_fwd", spec.le, spec.lo, spec.channels, S, nat.ptr(xtab), nat.ptr(species),
+             nat.ptr(sh), nat.ptr(h3), nat.ptr(W4), _w(spec), nat.ptr(mask), nat.ptr(topo.src), N, E,
+             nat.ptr(topo.by_dst.ptr), nat.ptr(topo.by_dst.order), nat.ptr(topo.dst_rows), nat.ptr(rows),
+             nat.ptr(out), nat.ptr(ws), nbytes, nat.stream_of(sh))
+    _timing.end(tok)
+    return out
+
+
+def _species_bwd_raw(spec, topo, xtab, species, sh, h3, t3, W4, mask, go, rows):
+    """(dsh, dr) of the species form for the cotangent go."""
+    N, E, S = species.shape[0], sh.shape[0], xtab.shape[0]
+    dsh, dr = torch.empty_like(sh), sh.new_empty(E)
+    ws, nbytes = _species_ws(spec, S, N, sh.device)
+    tok = _timing.begin(f"species_bwd[{spec.le}C{spec.channels}S{S}]")
+    nat.call("ictc_species_message_bwd", spec.le, spec.lo, spec.channels, S, nat.ptr(xtab), nat.ptr(species),
+             nat.ptr(sh), nat.ptr(h3), nat.ptr(t3), nat.ptr(W4), _w(spec), nat.ptr(mask), nat.ptr(topo.src),
+             N, E, nat.ptr(topo.by_dst.ptr), nat.ptr(topo.by_dst.order), nat.ptr(topo.dst_rows),
+             nat.ptr(rows), nat.ptr(go), nat.ptr(dsh), nat.ptr(dr), nat.ptr(ws), nbytes, nat.stream_of(sh))
+    _timing.end(tok)
+    return dsh, dr
+
+
+def _fused_fwd_raw(spec, topo, x, sh, h3, w4s, mask, rows):
+    N, E = x.shape[0], sh.shape[0]
+    out = x.new_empty(N, spec.out_components * spec.channels)
+    nat.call("ictc_msg_fused_fwd", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh),
+             nat.ptr(h3), nat.ptr(w4s), nat.ptr(mask), nat.ptr(topo.src), N, E, nat.ptr(topo.by_dst.ptr),
+             nat.ptr(topo.by_dst.order), nat.ptr(topo.dst_rows), nat.ptr(out), nat.ptr(rows), nat.stream_of(x))
+    return out
+
+
+def _fused_bwd_raw(spec, topo, x, sh, h3, t3, w4s, mask, go, need, rows):
+    """(dx, dsh, dr) of the fused message; need = (dx wanted, dsh wanted)."""
+    N, E = x.shape[0], sh.shape[0]
+    dx = torch.empty_like(x) if need[0] else None
+    dsh = torch.empty_like(sh) if need[1] else None
+    dr = sh.new_empty(E)
+    sp = topo.by_src if need[0] else None
+    nat.call("ictc_msg_fused_bwd_tangent", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh),
+             nat.ptr(h3), nat.ptr(t3), nat.ptr(w4s), nat.ptr(mask), nat.ptr(topo.src), nat.ptr(topo.dst),
+             N, E, nat.ptr(topo.by_dst.ptr), nat.ptr(topo.by_dst.order),
+             nat.ptr(sp.ptr) if sp else None, nat.ptr(sp.order) if sp else None, nat.ptr(topo.dst_rows),
+             nat.ptr(topo.src_rows), nat.ptr(go), nat.ptr(dx), nat.ptr(dsh), nat.ptr(dr),
+             nat.ptr(rows), nat.stream_of(x))
+    return dx, dsh, dr
 
 
 def _species_ws(spec, S, N, device):
@@ -878,19 +925,9 @@ class FusedRadialMessage(torch.autograd.Function):
         ctx.spec, ctx.topo, ctx.mask, ctx.cfg, ctx.w4s = spec, topo, mask, cfg, w4s
         x, sh, rc = _c(x), _c(sh), _c(r.detach())
         Ws = [_c(w.detach()) for w in (W1, W2, W3, W4)]
-        E = rc.shape[0]
-        rg = _c(topo.gate_input(rc))     # one row per edge pair
+        h3, t3 = _mlp_tangent_raw(topo.gate_input(rc), Ws, cfg)     # one row per edge pair
         ctx.rows = topo.gate_rows
-        h3, t3 = rc.new_empty(rg.shape[0], 64), rc.new_empty(rg.shape[0], 64)
-        nat.call("ictc_radial_mlp_tangent_fwd", nat.ptr(rg), rg.shape[0], 8, 64, float(cfg[0]), int(cfg[1]),
-                 nat.ptr(Ws[0]), nat.ptr(Ws[1]), nat.ptr(Ws[2]), float(cfg[2]), nat.ptr(h3), nat.ptr(t3),
-                 nat.stream_of(rc))
-        N = x.shape[0]
-        out = x.new_empty(N, spec.out_components * spec.channels)
-        nat.call("ictc_msg_fused_fwd", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh),
-                 nat.ptr(h3), nat.ptr(w4s), nat.ptr(mask), nat.ptr(topo.src), N, E, nat.ptr(topo.by_dst.ptr),
-                 nat.ptr(topo.by_dst.order), nat.ptr(topo.dst_rows), nat.ptr(out), nat.ptr(ctx.rows),
-                 nat.stream_of(x))
+        out = _fused_fwd_raw(spec, topo, x, sh, h3, w4s, mask, ctx.rows)
         ctx.save_for_backward(x, sh, rc, *Ws, h3, t3)
         return out
 
@@ -912,17 +949,7 @@ class FusedRadialMessage(torch.autograd.Function):
             return (dx, dsh, dr, *dW, None, None, None, None, None)
         if not any(needs[:3]):
             return (None,) * 12
-        N, E = x.shape[0], sh.shape[0]
-        dx = torch.empty_like(x) if needs[0] else None
-        dsh = torch.empty_like(sh) if needs[1] else None
-        dr = sh.new_empty(E)
-        sp = topo.by_src if needs[0] else None
-        nat.call("ictc_msg_fused_bwd_tangent", spec.li, spec.le, spec.lo, spec.channels, nat.ptr(x), nat.ptr(sh),
-                 nat.ptr(h3), nat.ptr(t3), nat.ptr(ctx.w4s), nat.ptr(mask), nat.ptr(topo.src), nat.ptr(topo.dst),
-                 N, E, nat.ptr(topo.by_dst.ptr), nat.ptr(topo.by_dst.order),
-                 nat.ptr(sp.ptr) if sp else None, nat.ptr(sp.order) if sp else None, nat.ptr(topo.dst_rows),
-                 nat.ptr(topo.src_rows), nat.ptr(go), nat.ptr(dx), nat.ptr(dsh), nat.ptr(dr),
-                 nat.ptr(ctx.rows), nat.stream_of(x))
+        dx, dsh, dr = _fused_bwd_raw(spec, topo, x, sh, h3, t3, ctx.w4s, mask, go, needs[:2], ctx.rows)
         return (dx, dsh, dr if needs[2] else None, None, None, None, None, None, None, None, None, None)
 
 

@@ -320,24 +320,10 @@ class PureCartesianICTDFix(nn.Module):
         from ictc_o3.ops.activation import radial_embedding
         return radial_embedding(r, self.max_radius, self.number_of_basis, self.polynomial_cutoff_p)
 
-    def forward(self, pos, A, batch, edge_src, edge_dst, edge_shifts, cell, *, topology=None, second_order=True,
-                forces_only=False):
-        """Per-atom energies [N, 1].
-
-        forces_only=True (with second_order=False) tells the fused path that the
-        backward will ask for position gradients and no parameter gradients: the
-        radial gates are then written with their derivative along r, and the
-        message adjoint forms dE/dr without the gate gradient.  A backward that
-        does ask for parameter gradients stays correct (it takes the ordinary
-        route), only slower.
-
-        second_order=False allows the fused radial-MLP kernel, whose adjoint
-        supports first derivatives only (forces, parameter gradients); the
-        default keeps every operator differentiable to second order.
-        """
-        N = pos.shape[0]
+    def species_indices(self, A):
+        """Compact species [N] of the atomic numbers, validated (backbone.py:996-1009)."""
         A_long = A.long()
-        # species validation of backbone.py:996-1009 (skip_input_validation drops its host syncs).  The
+        # skip_input_validation drops the validation's host syncs.  The
         # same live tensor object with an unchanged version counter is validated once: MD and training
         # loops pass one atomic-number tensor every step, and a sync per step would stall the launches.
         seen = getattr(self, "_validated_z", None)
@@ -360,6 +346,25 @@ class PureCartesianICTDFix(nn.Module):
                 raise ValueError(f"Encountered atomic numbers without compact mapping: {bad}. "
                                  f"Configured atomic_numbers={self.atomic_numbers}")
             self._validated_z = (weakref.ref(A), A._version)
+        return species
+
+    def forward(self, pos, A, batch, edge_src, edge_dst, edge_shifts, cell, *, topology=None, second_order=True,
+                forces_only=False):
+        """Per-atom energies [N, 1].
+
+        forces_only=True (with second_order=False) tells the fused path that the
+        backward will ask for position gradients and no parameter gradients: the
+        radial gates are then written with their derivative along r, and the
+        message adjoint forms dE/dr without the gate gradient.  A backward that
+        does ask for parameter gradients stays correct (it takes the ordinary
+        route), only slower.
+
+        second_order=False allows the fused radial-MLP kernel, whose adjoint
+        supports first derivatives only (forces, parameter gradients); the
+        default keeps every operator differentiable to second order.
+        """
+        N = pos.shape[0]
+        species = self.species_indices(A)
         if topology is None:
             # spatial row order for one periodic system; batched graphs keep index order (their
             # atoms are contiguous per graph, and the graphs' coordinates overlap)

@@ -53,6 +53,21 @@ def create_model(*, channels=64, lmax=3, edge_lmax=None, num_interactions=2, cor
     return model.to(device=device)
 
 
+def _graph_energies(selected, batch, cell):
+    """Per-graph energies in FP64 without atomics (deterministic, contention free)."""
+    if cell.shape[0] == 1:
+        return selected.double().sum().reshape(1)
+    if selected.is_cuda and selected.dtype == torch.float32:
+        from ictc_o3.ops.linear import graph_sum
+        graphs, n = cell.shape[0], selected.shape[0]
+        # Many small graphs: the contiguous-batch form is O(N + graphs) instead of O(graphs * N); the
+        # one host read deciding it is paid only where the quadratic form would cost more.
+        ordered = graphs > 64 and n > 1 and bool((batch[1:] >= batch[:-1]).all())
+        return graph_sum(selected, batch, graphs, batch_sorted=ordered)
+    onehot = torch.nn.functional.one_hot(batch, cell.shape[0]).to(torch.float64)
+    return onehot.t() @ selected.double()
+
+
 def energy_and_forces(model, positions, atomic_numbers, batch, edge_src, edge_dst, edge_shifts, cell, *,
                       training=False, owned_mask=None, topology=None):
     """Energy [B], forces [N,3], atomic_energy [N] of a prebuilt graph (runtime.py:86-113).
@@ -70,25 +85,20 @@ def energy_and_forces(model, positions, atomic_numbers, batch, edge_src, edge_ds
         raise ValueError("Atomic numbers and graph batch must have shape [N]")
     if owned_mask is not None and (owned_mask.shape != (n,) or owned_mask.requires_grad):
         raise ValueError("owned_mask must be a fixed [N] tensor")
+    if not training:
+        from mace_ictc.hp.direct import energy_forces
+        done = energy_forces(model, positions, atomic_numbers, batch, edge_src, edge_dst, edge_shifts, cell, topology,
+                             owned_mask, _graph_energies)
+        if done is not None:
+            atomic, energy64, force = done
+            return {"energy": energy64.to(atomic.dtype), "forces": force, "atomic_energy": atomic}
     with torch.enable_grad():
         pos = positions if positions.requires_grad else positions.detach().requires_grad_(True)
         output = model(pos, atomic_numbers, batch, edge_src, edge_dst, edge_shifts, cell, topology=topology,
                        second_order=training, forces_only=not training)
         atomic = (output[0] if isinstance(output, tuple) else output).reshape(n)
         selected = atomic if owned_mask is None else atomic * owned_mask.to(atomic)
-        # per-graph sums in FP64 without atomics (deterministic, contention free)
-        if cell.shape[0] == 1:
-            energy64 = selected.double().sum().reshape(1)
-        elif selected.is_cuda and selected.dtype == torch.float32:
-            from ictc_o3.ops.linear import graph_sum
-            graphs = cell.shape[0]
-            # Many small graphs: the contiguous-batch form is O(N + graphs) instead of O(graphs * N); the
-            # one host read deciding it is paid only where the quadratic form would cost more.
-            ordered = graphs > 64 and n > 1 and bool((batch[1:] >= batch[:-1]).all())
-            energy64 = graph_sum(selected, batch, graphs, batch_sorted=ordered)
-        else:
-            onehot = torch.nn.functional.one_hot(batch, cell.shape[0]).to(torch.float64)
-            energy64 = onehot.t() @ selected.double()
+        energy64 = _graph_energies(selected, batch, cell)
         force = -torch.autograd.grad(energy64.sum() + pos.sum() * 0.0, pos, create_graph=training,
                                      retain_graph=training)[0]
         energy = energy64.to(atomic.dtype)
