@@ -16,8 +16,8 @@ component order (component k of degree l sits at l*l + m):
   dy    dy[j] += sum_p gw[p] sum C_p x[m1] go[k]
   dg    dg[p]  = sum_k go[k] sum C_p x[m1] y[m2]
   dydg  dy and dg of the same x in one pass
-  dxdydg dx, dy and dg in one pass, factorised through V_p[i][j] = sum_k C go[k]
-  dydg_v, dx_v  the same factorisation for dy + dg alone and for dx alone
+  adjoint  dx, dy and dg path by path, factorised through V_p[i][j] = sum_k C go[k]
+  dx_v     the same factorisation for dx alone
 
 The sums are grouped so that the lane-varying operand meets the CG literal
 first: B_jk = sum_i C x[i] costs one VALU op per nonzero, and the per-edge
@@ -203,40 +203,45 @@ def tp_struct(li, le, lo):
     for p, i, j, k, v in ent:
         by_pij.setdefault(p, {}).setdefault((i, j), []).append((k, v))
 
-    def factored(name, args, want_dx, want_dydg):
-        lines.append(f"  __device__ __forceinline__ static void {name}({args}) {{")
-        for p in range(P):
-            pairs = by_pij.get(p, {})
-            lines.append("    {")
-            for (i, j), ks in sorted(pairs.items()):
-                lines.append(f"      const float v{i}_{j} = {' + '.join(f'{f(v)} * go[{k}]' for k, v in ks)};")
-            rows = {}
-            cols = {}
-            for (i, j) in sorted(pairs):
-                rows.setdefault(i, []).append(j)
-                cols.setdefault(j, []).append(i)
-            if want_dx:
-                for i, js in sorted(rows.items()):
-                    lines.append(f"      d[{i}] = fmaf(gw[{p}], {' + '.join(f'v{i}_{j} * y[{j}]' for j in js)}, d[{i}]);")
-            if want_dydg:
-                tl = []
-                for j, is_ in sorted(cols.items()):
-                    lines.append(f"      const float t{j} = {' + '.join(f'v{i}_{j} * x[{i}]' for i in is_)};")
-                    lines.append(f"      dyv[{j}] = fmaf(gw[{p}], t{j}, dyv[{j}]);")
-                    tl.append(f"y[{j}] * t{j}")
-                lines.append(f"      dg[{p}] = {' + '.join(tl) if tl else '0.f'};")
-            lines.append(f"    }}{SB}")
-        lines.append("  }")
-
-    factored("dxdydg", "const float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ gw, "
-             "const float* __restrict__ go, float* __restrict__ d, float* __restrict__ dyv, float* __restrict__ dg",
-             True, True)
-    # dy and dg alone (x varies per edge, so nothing of dydg's B_jk(x) survives between edges)
-    factored("dydg_v", "const float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ gw, "
-             "const float* __restrict__ go, float* __restrict__ dyv, float* __restrict__ dg", False, True)
+    # dx, dy and dg path by path, on an edge e that holds its own cotangent row: e.gate(p) is the path's gate,
+    # e.dg(p, v) takes its gate gradient, and e.used(p) / e.used_out(k) say that the path's values (go[k]
+    # belongs to one path) have been read for the last time, so that the next edge's can load into their place.
+    # The barrier keeps those loads behind the path's products.
+    lines.append("  template <class E>")
+    lines.append("  __device__ __forceinline__ static void adjoint(const float* __restrict__ x, const float* __restrict__ y,"
+                 " E& e, float* __restrict__ d, float* __restrict__ dyv) {")
+    for p in range(P):
+        pairs = by_pij.get(p, {})
+        lines.append(f"    {{ const float g = e.gate({p});")
+        for (i, j), ks in sorted(pairs.items()):
+            lines.append(f"      const float v{i}_{j} = {' + '.join(f'{f(v)} * e.go[{k}]' for k, v in ks)};")
+        for i in sorted({i for i, _ in pairs}):
+            js = [j for a, j in sorted(pairs) if a == i]
+            lines.append(f"      d[{i}] = fmaf(g, {' + '.join(f'v{i}_{j} * y[{j}]' for j in js)}, d[{i}]);")
+        tl = []
+        for j in sorted({j for _, j in pairs}):
+            is_ = [i for i, b in sorted(pairs) if b == j]
+            lines.append(f"      const float t{j} = {' + '.join(f'v{i}_{j} * x[{i}]' for i in is_)};")
+            lines.append(f"      dyv[{j}] = fmaf(g, t{j}, dyv[{j}]);")
+            tl.append(f"y[{j}] * t{j}")
+        lines.append(f"      e.dg({p}, {' + '.join(tl) if tl else '0.f'});")
+        used = sorted({k for ks in pairs.values() for k, _ in ks})
+        lines.append(f"      e.used({p}); {' '.join(f'e.used_out({k});' for k in used)} }}")
+        lines.append("    __builtin_amdgcn_sched_barrier(0);")
+    lines.append("  }")
     # dx alone
-    factored("dx_v", "const float* __restrict__ y, const float* __restrict__ gw, const float* __restrict__ go, "
-             "float* __restrict__ d", True, False)
+    lines.append("  __device__ __forceinline__ static void dx_v(const float* __restrict__ y, const float* __restrict__ gw,"
+                 " const float* __restrict__ go, float* __restrict__ d) {")
+    for p in range(P):
+        pairs = by_pij.get(p, {})
+        lines.append("    {")
+        for (i, j), ks in sorted(pairs.items()):
+            lines.append(f"      const float v{i}_{j} = {' + '.join(f'{f(v)} * go[{k}]' for k, v in ks)};")
+        for i in sorted({i for i, _ in pairs}):
+            js = [j for a, j in sorted(pairs) if a == i]
+            lines.append(f"      d[{i}] = fmaf(gw[{p}], {' + '.join(f'v{i}_{j} * y[{j}]' for j in js)}, d[{i}]);")
+        lines.append(f"    }}{SB}")
+    lines.append("  }")
     lines.append("};")
     return "\n".join(lines)
 

@@ -137,6 +137,17 @@ __device__ __forceinline__ void load_row_stream(const float* __restrict__ base, 
   }
 }
 
+// A row as a buffer descriptor (wave-uniform base, `bytes` readable) and one component of it: the lane's byte
+// offset in a VGPR, the component's in an SGPR.  kStream: a row read once, as in load_row_stream.
+constexpr int kCached = 0, kStream = 2;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000);
+}
+template <int AUX>
+__device__ __forceinline__ float row_load(__amdgpu_buffer_rsrc_t row, int off, int component) {
+  return __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(row, off, component, AUX));
+}
+
 template <int N>
 __device__ __forceinline__ void zero_row(float* v) {
 #pragma unroll
@@ -714,12 +725,11 @@ __device__ __forceinline__ void store_dsh_dr(float* __restrict__ dsh_g, float* _
 }
 
 // This lane's share of the gate-tangent dot: sum_p dg[p] w[p] gdot[p] (dg unweighted, unmasked).
-// W: 1 / 0 = with / without the per-path weight, known at compile time; -1 = tested at run time.
-template <class T, int W = -1>
+template <class T>
 __device__ __forceinline__ float gate_tangent_dot(const Operands& a, const float* __restrict__ gdot, int64_t e, int c,
                                                   const float* gt, const float* dg) {
   float t = 0.f;
-  if (W == 1 || (W < 0 && a.weight)) {
+  if (a.weight) {
 #pragma unroll
     for (int p = 0; p < T::P; ++p) t += dg[p] * a.weight[p * a.channels + c] * gt[p];
   } else {
@@ -878,34 +888,10 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX, T::LI, T::LE, T::LO>::
 // the sender's own features are loaded once per row.  Row slot `rows` covers
 // the out-of-range tail segment of the source CSR and writes zero gate and
 // harmonic gradients for it (no feature row).
-// Waves per SIMD of the source-owned adjoint.  The gate-tangent form streams the
-// tangent rows as well; where the table allows 3 it runs better at 2, with fewer
-// receiver rows in flight (cfg4 layer-1 shape: 8.62 ms at 2, 9.6 ms at 3 with 13
-// spilled VGPRs).
-template <class T, bool TAN>
-constexpr int src_adjoint_waves() {
-  return (TAN && Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value == 3)
-             ? 2
-             : Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value;
-}
-
-// The gate-tangent form keeps two edges' cotangent, gate and gate-tangent rows in flight where it runs
-// at 2 waves per SIMD (up to 256 VGPRs) and the second set of rows is at most 57 values per lane
-// (NO + 2 P): at 60, the (1,3,3) and (3,1,3) triples spill.
-template <class T, bool TAN>
-constexpr bool src_adjoint_pipelined() {
-  return TAN && src_adjoint_waves<T, TAN>() == 2 && T::NO + 2 * T::P <= 57;
-}
-
-// TAN: as in msg_bwd_edge_kernel, dr from gdot in place of the gate gradient.
-// W: the per-path weight a.weight is set (chosen at launch).  One loop per kernel: with both forms in one
-// kernel they share one register allocation, and the gate-tangent form of Tp<2,2,2> spilled 15 VGPRs
-// (226 without a spill for the unweighted form alone).
-template <class T, bool TAN, bool W = false>
-__global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd_src_kernel(
+template <class T>
+__global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value)) void msg_bwd_src_kernel(
     Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx,
-    float* __restrict__ dsh, float* __restrict__ dsh_part, float* __restrict__ dgates, const float* __restrict__ gdot,
-    float* __restrict__ dr, float* __restrict__ dr_part, int parts) {
+    float* __restrict__ dsh, float* __restrict__ dsh_part, float* __restrict__ dgates, int parts) {
   const RowGroup rg = row_group_y_xcd();
   const RowShare rs = row_share(scsr, rg.row, a.rows + 1, a.rows, parts);
   if (parts == 1 && !rs.valid) return;
@@ -915,70 +901,10 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float* dsh_g = group_target(dsh, dsh_part, rg.group, a.edges, T::NY);
-  float* dr_g = rg.group > 0 ? dr_part + (int64_t)(rg.group - 1) * a.edges : dr;
   float xv[T::NX], d[T::NX];
   if (active && rs.valid && !tail) load_row<T::NX>(a.x + n * (int64_t)(T::NX * C), C, c, xv);
   else zero_row<T::NX>(xv);
   zero_row<T::NX>(d);
-  if constexpr (src_adjoint_pipelined<T, TAN>()) {
-    // Two edges in flight: the cotangent, gate and gate-tangent rows of edge i + 1 load while edge i
-    // computes (2 waves per SIMD leave room for the second set of rows).  Per-edge arithmetic is that
-    // of the unpipelined form, operand for operand.
-    auto run = [&](auto weighted) {
-    for (int32_t pos = beg; pos < end; pos += kWave) {
-      const int32_t count = min(end - pos, kWave);
-      Chunk<T> ch;
-      stage_chunk<T>(a, dst, scsr.order, pos, count, ch);
-      float go0[T::NO], gr0[T::P], gt0[T::P], go1[T::NO], gr1[T::P], gt1[T::P];
-      auto fetch = [&](int i, float* go, float* gr, float* gt) {
-        const int64_t r = lane_i(ch.peer, i), row = lane_i(ch.row, i);
-        load_row<T::NO>(grad + r * (int64_t)(T::NO * C), C, c, go);
-        load_row_stream<T::P>(a.gates + row * (int64_t)(T::P * C), C, c, gr);
-        load_row_stream<T::P>(gdot + row * (int64_t)(T::P * C), C, c, gt);
-      };
-      auto consume = [&](int i, const float* go, const float* gr, const float* gt) {
-        const int64_t e = lane_i(ch.e, i);
-        const float m = lane_f(ch.m, i);
-        float y[T::NY], dyv[T::NY], gw[T::P], dg[T::P];
-#pragma unroll
-        for (int j = 0; j < T::NY; ++j) {
-          y[j] = lane_f(ch.y[j], i);
-          dyv[j] = 0.f;
-        }
-        float dgt = 0.f;
-        if (active) {
-#pragma unroll
-          for (int p = 0; p < T::P; ++p) gw[p] = gr[p];
-          if constexpr (W) {
-#pragma unroll
-            for (int p = 0; p < T::P; ++p) gw[p] *= a.weight[p * C + c];
-          }
-#pragma unroll
-          for (int p = 0; p < T::P; ++p) gw[p] *= m;
-          if (dsh) {
-            T::dxdydg(xv, y, gw, go, d, dyv, dg);   // (the tail row's d is never stored)
-          } else {
-            if (!tail) T::dx_v(y, gw, go, d);
-            T::dg(xv, y, go, dg);
-          }
-          dgt = m * gate_tangent_dot<T, W ? 1 : 0>(a, gdot, e, c, gt, dg);
-        }
-        store_dsh_dr<T::NY>(dsh_g, dr_g, e, dyv, dgt);
-      };
-      if (active) fetch(0, go0, gr0, gt0);
-      for (int i = 0; i < count; i += 2) {
-        if (active && i + 1 < count) fetch(i + 1, go1, gr1, gt1);
-        consume(i, go0, gr0, gt0);
-        if (i + 1 >= count) break;
-        if (active && i + 2 < count) fetch(i + 2, go0, gr0, gt0);
-        consume(i + 1, go1, gr1, gt1);
-      }
-    }
-    };
-    run(Flag<W>{});
-    store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);
-    return;
-  }
   // An out-of-range receiver contributes zero (mask 0, row 0 read).
   for (int32_t pos = beg; pos < end; pos += kWave) {
     const int32_t count = min(end - pos, kWave);
@@ -993,21 +919,6 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd
       for (int j = 0; j < T::NY; ++j) {
         y[j] = lane_f(ch.y[j], i);
         dyv[j] = 0.f;
-      }
-      float dgt = 0.f;
-      if (TAN && active) {
-        float go[T::NO], gw[T::P], gt[T::P], dg[T::P];
-        load_row<T::NO>(grad + r * (int64_t)(T::NO * C), C, c, go);
-        load_gw<T, true>(a, lane_i(ch.row, i), c, m, gw);
-        load_row_stream<T::P>(gdot + lane_i(ch.row, i) * (int64_t)(T::P * C), C, c, gt);
-        if (!tail) T::dx_v(y, gw, go, d);
-        if (dsh) T::dydg(xv, y, gw, go, dyv, dg);
-        else T::dg(xv, y, go, dg);
-        dgt = m * gate_tangent_dot<T>(a, gdot, e, c, gt, dg);
-      }
-      if (TAN) {
-        store_dsh_dr<T::NY>(dsh_g, dr_g, e, dyv, dgt);
-        continue;
       }
       if (active) {
         float go[T::NO], gw[T::P], dg[T::P];
@@ -1032,6 +943,106 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, TAN>())) void msg_bwd
         const int j = wave_sums_slot();
         if (j >= 0 && j < T::NY) dsh_g[e * T::NY + j] = v;
       }
+    }
+  }
+  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);
+}
+
+// One edge of the source-owned gate-tangent adjoint: its cotangent, gate and gate-tangent values, and the rows of
+// the next edge.  An edge is NO + 2 P values a lane; with the next one in a second set of registers the pass took
+// 226-256 VGPRs at (2,2,2) and did not fit two waves a SIMD at (2,3,3), which read its rows in two kernels instead.
+// T::adjoint works path by path, and a path's values are read by no later path: the next edge's load into their
+// registers at once (used, used_out) and have the rest of this edge to arrive.  One set of registers carries the
+// loads ahead: 128 VGPRs without spills at (2,2,2), 198 at (2,3,3), 253 at (3,3,3).
+// 206 k edges, C128, (2,3,3): receiver-owned pass 889 us + feature pass 797 us -> 1,060 us in one.
+// 5.26 M edges, C64, (2,2,2): 7.97 -> 7.95 ms (four waves a SIMD in place of two; the time there is neither
+// latency nor order: any order of a source's edges gives the same, and the clock falls with the traffic).
+// W: the per-path weight is set (wt holds it).
+template <class T, bool W>
+struct RollingEdge {
+  float go[T::NO], gr[T::P], gt[T::P], wt[W ? T::P : 1];
+  float mask, dgt;
+  __amdgpu_buffer_rsrc_t next_go, next_gr, next_gt;
+  int off, pitch;
+  __device__ __forceinline__ float gate(int p) const { return (W ? gr[p] * wt[p] : gr[p]) * mask; }
+  __device__ __forceinline__ void dg(int p, float v) { dgt += (W ? v * wt[p] : v) * gt[p]; }
+  __device__ __forceinline__ void used(int p) {
+    gr[p] = row_load<kStream>(next_gr, off, p * pitch);
+    gt[p] = row_load<kStream>(next_gt, off, p * pitch);
+  }
+  __device__ __forceinline__ void used_out(int k) { go[k] = row_load<kCached>(next_go, off, k * pitch); }
+};
+
+// Waves per SIMD of the gate-tangent source-owned adjoint: what the edge's values and the row sums leave room for
+// without spills of the unweighted form ((1,3,3), 60 edge values, spills 25 at 4).
+template <class T, bool W>
+constexpr int src_tangent_waves() {
+  constexpr int edge = T::NO + (W ? 3 : 2) * T::P, live = edge + 2 * T::NX + T::NY;
+  return edge <= 57 && live <= 84 ? 4 : live <= 110 ? 3 : 2;
+}
+
+// Gate-tangent form: dr[e] = sum over paths and channels of (gate gradient) * gdot in place of the gate gradient.
+template <class T, bool W>
+__global__ __launch_bounds__(kBlock, (src_tangent_waves<T, W>())) void msg_bwd_src_tangent_kernel(
+    Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx,
+    float* __restrict__ dsh, float* __restrict__ dsh_part, const float* __restrict__ gdot, float* __restrict__ dr,
+    float* __restrict__ dr_part, int parts) {
+  const RowGroup rg = row_group_y_xcd();
+  const RowShare rs = row_share(scsr, rg.row, a.rows + 1, a.rows, parts);
+  if (parts == 1 && !rs.valid) return;
+  const int64_t n = rs.n;
+  const int32_t beg = rs.beg, end = rs.end;
+  const bool tail = n == a.rows;
+  const int C = a.channels, c = 64 * rg.group + lane_id();
+  const bool active = c < C;
+  float* dsh_g = group_target(dsh, dsh_part, rg.group, a.edges, T::NY);
+  float* dr_g = rg.group > 0 ? dr_part + (int64_t)(rg.group - 1) * a.edges : dr;
+  float xv[T::NX], d[T::NX];
+  if (active && rs.valid && !tail) load_row<T::NX>(a.x + n * (int64_t)(T::NX * C), C, c, xv);
+  else zero_row<T::NX>(xv);
+  zero_row<T::NX>(d);
+  RollingEdge<T, W> ed;
+  ed.off = c * 4, ed.pitch = C * 4;
+  if constexpr (W) {
+    if (active) load_row<T::P>(a.weight, C, c, ed.wt);
+    else zero_row<T::P>(ed.wt);
+  }
+  // An out-of-range receiver contributes zero (mask 0, row 0 read).
+  for (int32_t pos = beg; pos < end; pos += kWave) {
+    const int32_t count = min(end - pos, kWave);
+    Chunk<T> ch;
+    stage_chunk<T>(a, dst, scsr.order, pos, count, ch);
+    // rows of edge i; past the chunk's last edge, rows of no bytes (their loads return 0 and read nothing)
+    auto point = [&](int i) {
+      const int j = min(i, count - 1), live = i < count ? C * 4 : 0;
+      const int64_t r = lane_i(ch.peer, j), row = lane_i(ch.row, j);
+      ed.next_go = row_rsrc(grad + r * (int64_t)(T::NO * C), T::NO * live);
+      ed.next_gr = row_rsrc(a.gates + row * (int64_t)(T::P * C), T::P * live);
+      ed.next_gt = row_rsrc(gdot + row * (int64_t)(T::P * C), T::P * live);
+    };
+    point(0);
+    if (active) {
+#pragma unroll
+      for (int p = 0; p < T::P; ++p) ed.used(p);
+#pragma unroll
+      for (int k = 0; k < T::NO; ++k) ed.used_out(k);
+    }
+    for (int i = 0; i < count; ++i) {
+      const int64_t e = lane_i(ch.e, i);
+      point(i + 1);
+      ed.pitch = __builtin_amdgcn_readfirstlane(C * 4);
+      // Component offsets are formed at their loads: kept across edges they take up to 120 SGPRs, spilled to VGPRs.
+      asm volatile("" : "+s"(ed.pitch));
+      ed.mask = lane_f(ch.m, i);
+      ed.dgt = 0.f;
+      float y[T::NY], dyv[T::NY];
+#pragma unroll
+      for (int j = 0; j < T::NY; ++j) {
+        y[j] = lane_f(ch.y[j], i);
+        dyv[j] = 0.f;
+      }
+      if (active) T::adjoint(xv, y, ed, d, dyv);   // (the tail row's d is never stored)
+      store_dsh_dr<T::NY>(dsh_g, dr_g, e, dyv, ed.mask * ed.dgt);
     }
   }
   store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);

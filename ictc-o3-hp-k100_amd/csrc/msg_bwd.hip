@@ -18,8 +18,8 @@ struct MsgBwd {
     // One source-owned pass for all three (rows + 1 slots: the last covers the out-of-range tail) where it
     // keeps 2 waves per SIMD; the P17 shapes need the register room of two separate passes.
     if (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value >= 2 && dx && (dsh || dg)) {
-      hipLaunchKernelGGL((msg_bwd_src_kernel<T, false>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
-                         0, st, a, dst, scsr, grad, dx, dsh, ws, dg, nullptr, nullptr, nullptr, sum);
+      hipLaunchKernelGGL((msg_bwd_src_kernel<T>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
+                         0, st, a, dst, scsr, grad, dx, dsh, ws, dg, sum);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
       if (dsh) return launch_group_sum(dsh, ws, a.edges * T::NY, G - 1, st);

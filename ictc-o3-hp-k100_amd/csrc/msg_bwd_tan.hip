@@ -19,13 +19,14 @@ struct MsgBwdTan {
     const int G = channel_groups(a.channels), sum = sum_parts(a.rows, G, kSourceSumWaves);
     float* ws_dr = ws ? ws + (int64_t)(G - 1) * a.edges * T::NY : nullptr;
     hipError_t err;
-    if (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value >= 2 && dx) {
+    if (dx) {
+      const dim3 grid(blocks_for((a.rows + 1) * sum), G);
       if (a.weight)
-        hipLaunchKernelGGL((msg_bwd_src_kernel<T, true, true>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
-                           0, st, a, dst, scsr, grad, dx, dsh, ws, nullptr, gdot, dr, ws_dr, sum);
+        hipLaunchKernelGGL((msg_bwd_src_tangent_kernel<T, true>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx,
+                           dsh, ws, gdot, dr, ws_dr, sum);
       else
-        hipLaunchKernelGGL((msg_bwd_src_kernel<T, true, false>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
-                           0, st, a, dst, scsr, grad, dx, dsh, ws, nullptr, gdot, dr, ws_dr, sum);
+        hipLaunchKernelGGL((msg_bwd_src_tangent_kernel<T, false>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx,
+                           dsh, ws, gdot, dr, ws_dr, sum);
       if ((err = hipGetLastError()) != hipSuccess) return err;
     } else {
       const int parts = row_parts(a.rows + 1, G);
@@ -36,11 +37,6 @@ struct MsgBwdTan {
         hipLaunchKernelGGL((msg_bwd_edge_kernel<T, true, false>), dim3(blocks_for((a.rows + 1) * parts), G),
                            dim3(kBlock), 0, st, a, src, dcsr, grad, dsh, ws, nullptr, parts, gdot, dr, ws_dr);
       if ((err = hipGetLastError()) != hipSuccess) return err;
-      if (dx) {
-        hipLaunchKernelGGL((msg_bwd_x_kernel<T>), dim3(blocks_for(a.rows * sum), G), dim3(kBlock),
-                           bwd_x_lds_cap<T>(a.rows), st, a, dst, scsr, grad, dx, sum);
-        if ((err = hipGetLastError()) != hipSuccess) return err;
-      }
     }
     if (dsh && (err = launch_group_sum(dsh, ws, a.edges * T::NY, G - 1, st)) != hipSuccess) return err;
     return launch_group_sum(dr, ws_dr, a.edges, G - 1, st);
