@@ -212,7 +212,7 @@ constexpr int kMaxGroups = 4;
 // highest of 4, 3, 2, 1 at which the kernel compiles without register spills,
 // found by tune_occupancy.py and recorded in ictc_occupancy.h.
 enum KernelKind {
-  kEdgeFwd, kEdgeBwd, kMsgFwd, kMsgBwdEdge, kMsgBwdX, kEdgeSecond, kMsgFwd2, kMsgBwdEdge2, kMsgBwdX2, kMsgBwdSrc
+  kEdgeFwd, kEdgeBwd, kMsgFwd, kMsgBwdEdge, kMsgBwdX, kEdgeSecond, kMsgFwd2, kMsgBwdEdge2, kMsgBwdX2
 };
 template <int K, int LI, int LE, int LO>
 struct Occupancy {
@@ -888,105 +888,64 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX, T::LI, T::LE, T::LO>::
 // the sender's own features are loaded once per row.  Row slot `rows` covers
 // the out-of-range tail segment of the source CSR and writes zero gate and
 // harmonic gradients for it (no feature row).
-template <class T>
-__global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value)) void msg_bwd_src_kernel(
-    Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx,
-    float* __restrict__ dsh, float* __restrict__ dsh_part, float* __restrict__ dgates, int parts) {
-  const RowGroup rg = row_group_y_xcd();
-  const RowShare rs = row_share(scsr, rg.row, a.rows + 1, a.rows, parts);
-  if (parts == 1 && !rs.valid) return;
-  const int64_t n = rs.n;
-  const int32_t beg = rs.beg, end = rs.end;
-  const bool tail = n == a.rows;
-  const int C = a.channels, c = 64 * rg.group + lane_id();
-  const bool active = c < C;
-  float* dsh_g = group_target(dsh, dsh_part, rg.group, a.edges, T::NY);
-  float xv[T::NX], d[T::NX];
-  if (active && rs.valid && !tail) load_row<T::NX>(a.x + n * (int64_t)(T::NX * C), C, c, xv);
-  else zero_row<T::NX>(xv);
-  zero_row<T::NX>(d);
-  // An out-of-range receiver contributes zero (mask 0, row 0 read).
-  for (int32_t pos = beg; pos < end; pos += kWave) {
-    const int32_t count = min(end - pos, kWave);
-    Chunk<T> ch;
-    stage_chunk<T>(a, dst, scsr.order, pos, count, ch);
-    for (int i = 0; i < count; ++i) {
-      const int64_t e = lane_i(ch.e, i);
-      const int64_t r = lane_i(ch.peer, i);
-      const float m = lane_f(ch.m, i);
-      float y[T::NY], dyv[T::NY];
-#pragma unroll
-      for (int j = 0; j < T::NY; ++j) {
-        y[j] = lane_f(ch.y[j], i);
-        dyv[j] = 0.f;
-      }
-      if (active) {
-        float go[T::NO], gw[T::P], dg[T::P];
-        load_row<T::NO>(grad + r * (int64_t)(T::NO * C), C, c, go);
-        load_gw<T>(a, lane_i(ch.row, i), c, m, gw);
-        if (!tail) T::dx_v(y, gw, go, d);
-        if (dsh && dgates) T::dydg(xv, y, gw, go, dyv, dg);
-        else if (dsh) T::dy(xv, gw, go, dyv);
-        else if (dgates) T::dg(xv, y, go, dg);
-        if (dgates) {
-#pragma unroll
-          for (int p = 0; p < T::P; ++p) dg[p] *= m;
-          if (a.weight) {
-#pragma unroll
-            for (int p = 0; p < T::P; ++p) dg[p] *= a.weight[p * C + c];
-          }
-          store_dg_row<T::P>(a, dgates + e * (int64_t)(T::P * C), C, c, dg);
-        }
-      }
-      if (dsh) {
-        const float v = wave_sums<T::NY>(dyv);
-        const int j = wave_sums_slot();
-        if (j >= 0 && j < T::NY) dsh_g[e * T::NY + j] = v;
-      }
-    }
-  }
-  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);
-}
+//
+// GRAD says what becomes of the gate gradient: nothing, stored, added to the row dgates holds, or contracted
+// against the gate tangents gdot (dr[e] = sum over paths and channels of it times gdot).
+enum GateGrad { kNoGrad, kStoreGrad, kAddGrad, kTangent };
 
-// One edge of the source-owned gate-tangent adjoint: its cotangent, gate and gate-tangent values, and the rows of
-// the next edge.  An edge is NO + 2 P values a lane; with the next one in a second set of registers the pass took
+// One edge of it: its cotangent and gate values, with kTangent its gate tangents and with kAddGrad its dgates row
+// (both in gt), and the rows of the next edge.  With kTangent an edge is NO + 2 P values a lane; with the next one in a second set of registers the pass took
 // 226-256 VGPRs at (2,2,2) and did not fit two waves a SIMD at (2,3,3), which read its rows in two kernels instead.
 // T::adjoint works path by path, and a path's values are read by no later path: the next edge's load into their
 // registers at once (used, used_out) and have the rest of this edge to arrive.  One set of registers carries the
 // loads ahead: 128 VGPRs without spills at (2,2,2), 198 at (2,3,3), 253 at (3,3,3).
-// 206 k edges, C128, (2,3,3): receiver-owned pass 889 us + feature pass 797 us -> 1,060 us in one.
+// 206 k edges, C128, (2,3,3): receiver-owned pass 889 us + feature pass 797 us -> 1,060 us in one (kTangent).
+// Forward and adjoint (kStoreGrad) of 68 k edges, C64, (3,3,3): 803 -> 530 us (the two passes ran at one wave a SIMD);
+// of 148 k edges, C64, (2,2,2): 400 -> 360 us (32 spilled VGPRs at 3 waves -> none at 4).
 // 5.26 M edges, C64, (2,2,2): 7.97 -> 7.95 ms (four waves a SIMD in place of two; the time there is neither
 // latency nor order: any order of a source's edges gives the same, and the clock falls with the traffic).
 // W: the per-path weight is set (wt holds it).
-template <class T, bool W>
+template <class T, GateGrad GRAD, bool W>
 struct RollingEdge {
-  float go[T::NO], gr[T::P], gt[T::P], wt[W ? T::P : 1];
+  static constexpr bool kTwo = GRAD == kAddGrad || GRAD == kTangent;   // a second [P] row per edge
+  float go[T::NO], gr[T::P], gt[kTwo ? T::P : 1], wt[W ? T::P : 1];
   float mask, dgt;
-  __amdgpu_buffer_rsrc_t next_go, next_gr, next_gt;
+  __amdgpu_buffer_rsrc_t next_go, next_gr, next_gt, dgates;
   int off, pitch;
   __device__ __forceinline__ float gate(int p) const { return (W ? gr[p] * wt[p] : gr[p]) * mask; }
-  __device__ __forceinline__ void dg(int p, float v) { dgt += (W ? v * wt[p] : v) * gt[p]; }
+  __device__ __forceinline__ void dg(int p, float v) {
+    if constexpr (GRAD == kTangent) {
+      dgt += (W ? v * wt[p] : v) * gt[p];
+    } else if constexpr (GRAD != kNoGrad) {
+      v *= mask;
+      if (W) v *= wt[p];
+      if constexpr (GRAD == kAddGrad) {
+        asm volatile("" : "+v"(v));   // the stored gate gradient, rounded, is what is added (no FMA with its product)
+        v = gt[p] + v;
+      }
+      __builtin_amdgcn_raw_buffer_store_b32((uint32_t)__float_as_int(v), dgates, off, p * pitch, 0);
+    }
+  }
   __device__ __forceinline__ void used(int p) {
     gr[p] = row_load<kStream>(next_gr, off, p * pitch);
-    gt[p] = row_load<kStream>(next_gt, off, p * pitch);
+    if constexpr (kTwo) gt[p] = row_load<kStream>(next_gt, off, p * pitch);
   }
   __device__ __forceinline__ void used_out(int k) { go[k] = row_load<kCached>(next_go, off, k * pitch); }
 };
 
-// Waves per SIMD of the gate-tangent source-owned adjoint: what the edge's values and the row sums leave room for
-// without spills of the unweighted form ((1,3,3), 60 edge values, spills 25 at 4).
-template <class T, bool W>
-constexpr int src_tangent_waves() {
-  constexpr int edge = T::NO + (W ? 3 : 2) * T::P, live = edge + 2 * T::NX + T::NY;
-  return edge <= 57 && live <= 84 ? 4 : live <= 110 ? 3 : 2;
+// Waves per SIMD of the source-owned adjoint: what the edge's values and the row sums leave room for without spills
+// of the unweighted form ((1,3,3) with kTangent, 60 edge values, spills 25 at 4).
+template <class T, GateGrad GRAD, bool W>
+constexpr int src_adjoint_waves() {
+  constexpr int edge = T::NO + (1 + RollingEdge<T, GRAD, W>::kTwo + W) * T::P, live = edge + 3 * T::NX + T::NY;
+  return edge <= 57 && live <= 93 ? 4 : live <= 126 ? 3 : 2;
 }
 
-// Gate-tangent form: dr[e] = sum over paths and channels of (gate gradient) * gdot in place of the gate gradient.
-template <class T, bool W>
-__global__ __launch_bounds__(kBlock, (src_tangent_waves<T, W>())) void msg_bwd_src_tangent_kernel(
+template <class T, GateGrad GRAD, bool W>
+__global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, GRAD, W>())) void msg_bwd_src_kernel(
     Operands a, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad, float* __restrict__ dx,
-    float* __restrict__ dsh, float* __restrict__ dsh_part, const float* __restrict__ gdot, float* __restrict__ dr,
-    float* __restrict__ dr_part, int parts) {
+    float* __restrict__ dsh, float* __restrict__ dsh_part, float* __restrict__ dgates, const float* __restrict__ gdot,
+    float* __restrict__ dr, float* __restrict__ dr_part, int parts) {
   const RowGroup rg = row_group_y_xcd();
   const RowShare rs = row_share(scsr, rg.row, a.rows + 1, a.rows, parts);
   if (parts == 1 && !rs.valid) return;
@@ -996,12 +955,12 @@ __global__ __launch_bounds__(kBlock, (src_tangent_waves<T, W>())) void msg_bwd_s
   const int C = a.channels, c = 64 * rg.group + lane_id();
   const bool active = c < C;
   float* dsh_g = group_target(dsh, dsh_part, rg.group, a.edges, T::NY);
-  float* dr_g = rg.group > 0 ? dr_part + (int64_t)(rg.group - 1) * a.edges : dr;
+  float* dr_g = GRAD == kTangent && rg.group > 0 ? dr_part + (int64_t)(rg.group - 1) * a.edges : dr;
   float xv[T::NX], d[T::NX];
   if (active && rs.valid && !tail) load_row<T::NX>(a.x + n * (int64_t)(T::NX * C), C, c, xv);
   else zero_row<T::NX>(xv);
   zero_row<T::NX>(d);
-  RollingEdge<T, W> ed;
+  RollingEdge<T, GRAD, W> ed;
   ed.off = c * 4, ed.pitch = C * 4;
   if constexpr (W) {
     if (active) load_row<T::P>(a.weight, C, c, ed.wt);
@@ -1018,7 +977,9 @@ __global__ __launch_bounds__(kBlock, (src_tangent_waves<T, W>())) void msg_bwd_s
       const int64_t r = lane_i(ch.peer, j), row = lane_i(ch.row, j);
       ed.next_go = row_rsrc(grad + r * (int64_t)(T::NO * C), T::NO * live);
       ed.next_gr = row_rsrc(a.gates + row * (int64_t)(T::P * C), T::P * live);
-      ed.next_gt = row_rsrc(gdot + row * (int64_t)(T::P * C), T::P * live);
+      if constexpr (GRAD == kTangent) ed.next_gt = row_rsrc(gdot + row * (int64_t)(T::P * C), T::P * live);
+      if constexpr (GRAD == kAddGrad)
+        ed.next_gt = row_rsrc(dgates + lane_i(ch.e, j) * (int64_t)(T::P * C), T::P * live);
     };
     point(0);
     if (active) {
@@ -1034,7 +995,8 @@ __global__ __launch_bounds__(kBlock, (src_tangent_waves<T, W>())) void msg_bwd_s
       // Component offsets are formed at their loads: kept across edges they take up to 120 SGPRs, spilled to VGPRs.
       asm volatile("" : "+s"(ed.pitch));
       ed.mask = lane_f(ch.m, i);
-      ed.dgt = 0.f;
+      if constexpr (GRAD == kTangent) ed.dgt = 0.f;
+      else if constexpr (GRAD != kNoGrad) ed.dgates = row_rsrc(dgates + e * (int64_t)(T::P * C), T::P * C * 4);
       float y[T::NY], dyv[T::NY];
 #pragma unroll
       for (int j = 0; j < T::NY; ++j) {
@@ -1042,10 +1004,16 @@ __global__ __launch_bounds__(kBlock, (src_tangent_waves<T, W>())) void msg_bwd_s
         dyv[j] = 0.f;
       }
       if (active) T::adjoint(xv, y, ed, d, dyv);   // (the tail row's d is never stored)
-      store_dsh_dr<T::NY>(dsh_g, dr_g, e, dyv, ed.mask * ed.dgt);
+      if constexpr (GRAD == kTangent) {
+        store_dsh_dr<T::NY>(dsh_g, dr_g, e, dyv, ed.mask * ed.dgt);
+      } else if (dsh) {
+        const float v = wave_sums<T::NY>(dyv);
+        const int j = wave_sums_slot();
+        if (j >= 0 && j < T::NY) dsh_g[e * T::NY + j] = v;
+      }
     }
   }
-  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail && dx);
+  store_row_sum<T::NX>(dx + n * (int64_t)(T::NX * C), C, c, d, parts, rs, rs.valid && !tail);
 }
 
 // ---------------------------------------------------------------------------

@@ -12,14 +12,24 @@ struct MsgBwd {
   const float* grad;
   float *dx, *dsh, *dg, *ws;
   hipStream_t st;
+  template <class T, GateGrad GRAD>
+  void src_pass(int G, int sum) {
+    const dim3 grid(blocks_for((a.rows + 1) * sum), G);
+    if (a.weight)
+      hipLaunchKernelGGL((msg_bwd_src_kernel<T, GRAD, true>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx, dsh, ws,
+                         dg, nullptr, nullptr, nullptr, sum);
+    else
+      hipLaunchKernelGGL((msg_bwd_src_kernel<T, GRAD, false>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx, dsh,
+                         ws, dg, nullptr, nullptr, nullptr, sum);
+  }
   template <class T>
   hipError_t run() {
     const int G = channel_groups(a.channels), sum = sum_parts(a.rows, G, kSourceSumWaves);
-    // One source-owned pass for all three (rows + 1 slots: the last covers the out-of-range tail) where it
-    // keeps 2 waves per SIMD; the P17 shapes need the register room of two separate passes.
-    if (Occupancy<kMsgBwdSrc, T::LI, T::LE, T::LO>::value >= 2 && dx && (dsh || dg)) {
-      hipLaunchKernelGGL((msg_bwd_src_kernel<T>), dim3(blocks_for((a.rows + 1) * sum), G), dim3(kBlock),
-                         0, st, a, dst, scsr, grad, dx, dsh, ws, dg, sum);
+    // One source-owned pass for all three (rows + 1 slots: the last covers the out-of-range tail).
+    if (dx && (dsh || dg)) {
+      if (dg && a.dg_acc) src_pass<T, kAddGrad>(G, sum);
+      else if (dg) src_pass<T, kStoreGrad>(G, sum);
+      else src_pass<T, kNoGrad>(G, sum);
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
       if (dsh) return launch_group_sum(dsh, ws, a.edges * T::NY, G - 1, st);

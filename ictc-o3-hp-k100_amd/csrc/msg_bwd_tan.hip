@@ -22,11 +22,11 @@ struct MsgBwdTan {
     if (dx) {
       const dim3 grid(blocks_for((a.rows + 1) * sum), G);
       if (a.weight)
-        hipLaunchKernelGGL((msg_bwd_src_tangent_kernel<T, true>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx,
-                           dsh, ws, gdot, dr, ws_dr, sum);
+        hipLaunchKernelGGL((msg_bwd_src_kernel<T, kTangent, true>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx,
+                           dsh, ws, nullptr, gdot, dr, ws_dr, sum);
       else
-        hipLaunchKernelGGL((msg_bwd_src_tangent_kernel<T, false>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx,
-                           dsh, ws, gdot, dr, ws_dr, sum);
+        hipLaunchKernelGGL((msg_bwd_src_kernel<T, kTangent, false>), grid, dim3(kBlock), 0, st, a, dst, scsr, grad, dx,
+                           dsh, ws, nullptr, gdot, dr, ws_dr, sum);
       if ((err = hipGetLastError()) != hipSuccess) return err;
     } else {
       const int parts = row_parts(a.rows + 1, G);

@@ -25,13 +25,9 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 UNITS = ["tp_edge.hip", "msg_fwd.hip", "msg_bwd.hip", "tp_second.hip", "msg_second_rcv.hip", "msg_second_src.hip"]
 KINDS = {"edge_fwd_kernel": "kEdgeFwd", "edge_bwd_kernel": "kEdgeBwd", "msg_fwd_kernel": "kMsgFwd",
          "msg_bwd_edge_kernel": "kMsgBwdEdge", "msg_bwd_x_kernel": "kMsgBwdX", "edge_second_kernel": "kEdgeSecond",
-         "msg_fwd2_kernel": "kMsgFwd2", "msg_bwd_edge2_kernel": "kMsgBwdEdge2", "msg_bwd_x2_kernel": "kMsgBwdX2",
-         "msg_bwd_src_kernel": "kMsgBwdSrc"}
+         "msg_fwd2_kernel": "kMsgFwd2", "msg_bwd_edge2_kernel": "kMsgBwdEdge2", "msg_bwd_x2_kernel": "kMsgBwdX2"}
 LEVELS = (4, 3, 2, 1)
 SPILL_BUDGET = 8
-# Measured exceptions (kernel, LI, LE, LO) -> waves per SIMD.  The fused source-owned message adjoint at
-# the cfg4 layer-1 shape runs 9.05 ms at 3 waves per SIMD (31 spilled VGPRs) against 9.26 ms at 2.
-MEASURED = {("msg_bwd_src_kernel", 2, 2, 2): 3}
 NAME = re.compile(r"Function Name: _ZN4ictc\d+(\w+?)INS_2TpILi(\d)ELi(\d)ELi(\d)E")
 
 
@@ -66,7 +62,6 @@ def main(path=None):
             # scratch without spills would be a stack array: never acceptable
             if spill <= SPILL_BUDGET and (scratch == 0 or spill > 0) and w > choice.get(key, 0):
                 choice[key] = w
-    choice.update(MEASURED)
     keys = {k for usage in results.values() for k in usage}
     lines = ["// Generated by tune_occupancy.py: minimum waves per SIMD per (kernel, degree triple),",
              f"// the highest of 4, 3, 2, 1 with at most {SPILL_BUDGET} spilled VGPRs.  Do not edit.", "#pragma once", ""]
