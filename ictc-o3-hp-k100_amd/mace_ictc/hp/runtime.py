@@ -6,7 +6,9 @@ polynomial cutoff p=5, no sqrt(num_basis) norm, frozen unit TP coefficients,
 first-layer scalar self connection, 16-wide final readout).  configure_model
 validates the reference keywords and reports the single MI355X plan.
 energy_and_forces evaluates E, F = -dE/dpos and per-atom energies; the
-per-graph energy sum is accumulated in FP64.
+per-graph energy sum is accumulated in FP64.  Without training=True the forces
+come from an explicit adjoint sweep (direct.py) where nothing could observe an
+autograd graph, from autograd otherwise.
 """
 from __future__ import annotations
 
