@@ -40,8 +40,10 @@ def _usage(unit: str, waves: int):
     for line in text.splitlines():
         m = NAME.search(line)
         if m:
-            key = (m.group(1), int(m.group(2)), int(m.group(3)), int(m.group(4)))
-            out[key] = [0, 0]
+            # (the source-owned message adjoint fixes its own count from its register sizes)
+            key = (m.group(1), int(m.group(2)), int(m.group(3)), int(m.group(4))) if m.group(1) in KINDS else None
+            if key is not None:
+                out[key] = [0, 0]
         elif key is not None and "VGPRs Spill:" in line:
             out[key][0] = int(line.split(":")[-1].split()[0])
         elif key is not None and "ScratchSize [bytes/lane]:" in line:
