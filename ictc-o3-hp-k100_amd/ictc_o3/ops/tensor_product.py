@@ -742,21 +742,17 @@ PAIR_GATES = True
 SOURCE_CSR_FROM_PAIRS = True
 
 
-def _fused_weight(fc, W4, spec):
-    """W4 folded with the path weight and split into the fused kernels' MFMA operand layout, cached on `fc`
-    per (storage, version) of the weights (the reference's _folded_weights, streamed_gate_message.py:23-47)."""
+def _fused_weight(W4, spec):
+    """W4 folded with the path weight and split into the fused kernels' MFMA operand layout (the reference's
+    _folded_weights, streamed_gate_message.py:23-47).  Formed on each call, one small launch: kept between calls it
+    would have to be found again by the weight's address and version counter, and neither tells of a write through
+    ``weight.data``, of a contiguous copy that takes a freed copy's address, or of another stream's pending launch."""
     tpw = spec.weight
-    key = (W4.data_ptr(), W4._version, str(W4.device),
-           None if tpw is None else (tpw.data_ptr(), tpw._version))
-    cached = getattr(fc, "_ictc_fused_w4", None)
-    if cached is not None and cached[0] == key:
-        return cached[1]
     W = _c(W4.detach())
     nbytes = int(nat.lib().ictc_fused_weight_bytes(spec.num_paths, spec.channels))
     out = torch.empty(nbytes // 4, dtype=torch.float32, device=W.device)
     nat.call("ictc_fused_weight_split", nat.ptr(W), None if tpw is None else nat.ptr(_c(tpw.detach())),
              spec.num_paths, spec.channels, nat.ptr(out), nbytes, nat.stream_of(W))
-    fc._ictc_fused_w4 = (key, out)
     return out
 
 
@@ -965,7 +961,7 @@ def radial_message(x, sh, r, fc, spec, topo, mask, cfg, basis_scale=1.0, species
     if species is not None and _species_ok(spec, x, species[0]):
         return SpeciesRadialMessage.apply(x, sh, r, *W, spec, topo, mask, cfg, species[0], species[1])
     if _fused_ok(spec, x):
-        w4s = _fused_weight(fc, W[-1], spec)
+        w4s = _fused_weight(W[-1], spec)
         return FusedRadialMessage.apply(x, sh, r, *W, spec, topo, mask, cfg, w4s)
     return RadialMessage.apply(x, sh, r, *W, spec, topo, mask, cfg)
 

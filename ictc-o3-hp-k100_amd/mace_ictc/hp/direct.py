@@ -140,7 +140,7 @@ class _Layer:
             return tpo._species_fwd_raw(spec, topo, self.xtab, self.species, Y, self.h3, self.Ws[3], mask, topo.gate_rows)
         self.x = packed_linear_raw(h, self.up_layout, self.up_w)
         if tpo._fused_ok(spec, self.x):
-            self.form, self.w4s = "fused", tpo._fused_weight(self.inter.fc, self.Ws[3], spec)
+            self.form, self.w4s = "fused", tpo._fused_weight(self.Ws[3], spec)
             self.h3, self.t3 = tpo._mlp_tangent_raw(topo.gate_input(r), self.Ws, self.cfg)
             return tpo._fused_fwd_raw(spec, topo, self.x, Y, self.h3, self.w4s, mask, topo.gate_rows)
         self.form = "gates"
