@@ -19,7 +19,7 @@ from torch.nn.modules import module as _module
 from ictc_o3.ops import tensor_product as tpo
 from ictc_o3.ops.activation import _silu
 from ictc_o3.ops.geometry import _vector_adjoint, edge_harmonics_adjoint_raw, edge_harmonics_raw, shift_vectors
-from ictc_o3.ops.linear import (_fast_ok, _species_apply, _weight_operand, degree_layout, packed_linear_adjoint_raw,
+from ictc_o3.ops.linear import (_fast_ok, _species_apply, degree_layout, packed_linear_adjoint_raw,
                                 packed_linear_raw, path_layout, species_order)
 from ictc_o3.ops.radial_mlp import (edge_linear_adjoint_raw, edge_linear_raw, fused_supported,
                                     radial_gates_tangent)
@@ -205,7 +205,7 @@ def energy_forces(model, pos, A, batch, edge_src, edge_dst, shifts, cell, topolo
     r, n, mask, Y = edge_harmonics_raw(pos, shift, topo, model.max_radius, model.ictd_fix_edge_lmax)
     from mace_ictc.hp.model import SILU_SCALE
     cfg = (float(model.max_radius), int(model.polynomial_cutoff_p), SILU_SCALE)
-    table = _weight_operand(model.node_embedding.weight, transpose=True)     # [S, C]
+    table = model.node_embedding.weight.detach().t().contiguous()     # [S, C]
     h = h0 = table.index_select(0, species)
     layers, atomic = [], None
     for i in range(model.num_interaction):

@@ -60,3 +60,14 @@ def test_last_radial_weight_of_the_fused_message(device, monkeypatch, change, tr
     change(lin.weight, (1.5 * lin.weight.detach()).clone(memory_format=torch.preserve_format))
     moved = rel_err(_check(monkeypatch, model, args, change.__name__), before)
     assert moved > 1e-2
+
+
+@pytest.mark.parametrize("change", [_in_place, _through_data, _new_storage])
+@pytest.mark.parametrize("S", [3, 5])
+def test_node_embedding(device, monkeypatch, change, S):
+    model, args = _model(device, S), _system(device, S)
+    w = model.node_embedding.weight
+    before = _check(monkeypatch, model, args, "as built")
+    change(w, -0.5 * w.detach())
+    moved = rel_err(_check(monkeypatch, model, args, change.__name__), before)
+    assert moved > 1e-2
