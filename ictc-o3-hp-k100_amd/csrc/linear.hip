@@ -300,9 +300,63 @@ int launch_bf16(const float* in, int64_t in_stride, float* out, int64_t out_stri
   return ICTC_OK;
 }
 
+// Transposes of several small matrices in one launch: block (x, y) turns the x-th 32 x 32 tile of matrix y through
+// LDS (odd pitch: no bank conflicts; both sides coalesced).  Launch-bound: the weights of a C128 model with degree-3
+// edges are 4 MB, and one copy kernel per matrix was 15 launches a step.
+constexpr int kTransposeMost = 64, kTransposeTile = 32;
+struct TransposeList {
+  const float* src[kTransposeMost];
+  float* dst[kTransposeMost];
+  int rows[kTransposeMost], cols[kTransposeMost];
+};
+__global__ __launch_bounds__(256) void transpose_kernel(TransposeList t) {
+  __shared__ float tile[kTransposeTile][kTransposeTile + 1];
+  const int k = blockIdx.y, rows = t.rows[k], cols = t.cols[k];
+  const int across = (cols + kTransposeTile - 1) / kTransposeTile;
+  const int r0 = (int)blockIdx.x / across * kTransposeTile, c0 = (int)blockIdx.x % across * kTransposeTile;
+  if (r0 >= rows) return;
+  const int i = threadIdx.x & 31, j0 = threadIdx.x >> 5;
+  for (int j = j0; j < kTransposeTile; j += 8)
+    if (r0 + j < rows && c0 + i < cols) tile[j][i] = t.src[k][(int64_t)(r0 + j) * cols + c0 + i];
+  __syncthreads();
+  for (int j = j0; j < kTransposeTile; j += 8)
+    if (c0 + j < cols && r0 + i < rows) t.dst[k][(int64_t)(c0 + j) * rows + r0 + i] = tile[i][j];
+}
+
 }  // namespace
 
 extern "C" {
+
+int ictc_transpose(int count, const float* const* src, const int* rows, const int* cols, float* const* dst,
+                   void* stream) {
+  if (count < 0 || (count > 0 && (!src || !rows || !cols || !dst)))
+    return fail(ICTC_ERR_ARGUMENT, "transpose: invalid arguments");
+  for (int k = 0; k < count; ++k)
+    if (rows[k] < 0 || cols[k] < 0 || rows[k] > (1 << 20) || cols[k] > (1 << 20) ||
+        ((int64_t)rows[k] * cols[k] > 0 && (!src[k] || !dst[k])))
+      return fail(ICTC_ERR_ARGUMENT, "transpose: null matrix, or a side outside 0..2^20");
+  for (int k0 = 0; k0 < count; k0 += kTransposeMost) {
+    TransposeList t{};
+    int64_t tiles = 0;
+    const int n = std::min(count - k0, kTransposeMost);
+    for (int k = 0; k < n; ++k) {
+      t.src[k] = src[k0 + k], t.dst[k] = dst[k0 + k];
+      t.rows[k] = rows[k0 + k], t.cols[k] = std::max(cols[k0 + k], 1);
+      if (cols[k0 + k] == 0) t.rows[k] = 0;
+      tiles = std::max(tiles, (int64_t)((t.rows[k] + kTransposeTile - 1) / kTransposeTile) *
+                                  ((t.cols[k] + kTransposeTile - 1) / kTransposeTile));
+    }
+    if (tiles == 0) continue;
+    hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)tiles, n), dim3(256), 0, (hipStream_t)stream, t);
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    char buf[256];
+    snprintf(buf, sizeof(buf), "ictc_transpose launch: %s", hipGetErrorString(e));
+    return fail(ICTC_ERR_RUNTIME, buf);
+  }
+  return ICTC_OK;
+}
 
 int ictc_packed_linear(int lmax, int channels_in, int channels_out, const float* in, int64_t in_stride,
                        const int* in_paths, const int64_t* in_offsets, float* out, int64_t out_stride,

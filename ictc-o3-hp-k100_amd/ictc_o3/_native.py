@@ -67,6 +67,7 @@ _SIGNATURES = {
     "ictc_sh_hvp": (_i, [_p, _p, _p, _i64, _i, _p, _p]),
     "ictc_silu": (_i, [_i, _p, _p, _p, ctypes.c_float, _i64, _p, _p]),
     "ictc_radial": (_i, [_i, _p, _p, _p, _i64, _i, ctypes.c_float, _i, _p, _p]),
+    "ictc_transpose": (_i, [_i, _p, _p, _p, _p, _p]),
     "ictc_packed_linear": (_i, [_i, _i, _i, _p, _i64, _p, _p, _p, _i64, _p, _p, _p, _p, _i64, _p]),
     "ictc_neighbors_workspace_bytes": (_i64, [_i64, _p]),
     "ictc_neighbors_count": (_i, [_p, _i64, _p, ctypes.c_double, _p, _p, _i64, _p, _p]),

@@ -306,7 +306,9 @@ def _packed_adjoint(x, ws, layout, dout, needs):
     """Input adjoint (needs[0]) and weight gradients (needs[1:]) of the packed linear for cotangent dout."""
     lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
     dout = dout if dout.is_contiguous() else dout.contiguous()
-    dx = packed_linear_adjoint_raw(dout, layout, ws) if needs[0] else None
+    dx = None
+    if needs[0]:
+        dx = packed_linear_adjoint_raw(dout, layout, [_weight_operand(w, transpose=True) for w in ws])
     dws = []
     N = x.shape[0]
     for l, (w, need) in enumerate(zip(ws, needs[1:])):
@@ -581,14 +583,26 @@ def path_layout(weights, counts, C, lmax, scale=1.0):
 
 
 def packed_linear_raw(x, layout, weights):
-    """The packed linear of a _PackedLinear layout (no autograd)."""
+    """The packed linear of a _PackedLinear layout with contiguous weights (no autograd)."""
     lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
-    return _packed_call(x, Ci, Co, lmax, pin, in_off, [1] * (lmax + 1), out_off, [_weight_operand(w) for w in weights],
-                        scales, (lmax + 1) ** 2 * Co)
+    return _packed_call(x, Ci, Co, lmax, pin, in_off, [1] * (lmax + 1), out_off, weights, scales, (lmax + 1) ** 2 * Co)
 
 
-def packed_linear_adjoint_raw(dout, layout, weights):
-    """Its input adjoint."""
+def packed_linear_adjoint_raw(dout, layout, transposed_weights):
+    """Its input adjoint, with the contiguous transposes of the weights."""
     lmax, Ci, Co, pin, in_off, out_off, scales, in_cols = layout
-    wt = [_weight_operand(w, transpose=True) for w in weights]
-    return _packed_call(dout, Co, Ci, lmax, [1] * (lmax + 1), out_off, pin, in_off, wt, scales, in_cols)
+    return _packed_call(dout, Co, Ci, lmax, [1] * (lmax + 1), out_off, pin, in_off, transposed_weights, scales, in_cols)
+
+
+def transposed(matrices):
+    """Contiguous transposes of contiguous float32 device matrices, in one launch."""
+    n, offs, total = len(matrices), [], 0
+    for m in matrices:
+        offs.append(total)
+        total += (m.numel() + 63) // 64 * 64   # the packed kernel reads 16-byte runs
+    buf = matrices[0].new_empty(total)
+    out = [buf[o:o + m.numel()].view(m.shape[1], m.shape[0]) for o, m in zip(offs, matrices)]
+    nat.call("ictc_transpose", n, (ctypes.c_void_p * n)(*[m.data_ptr() for m in matrices]),
+             (ctypes.c_int * n)(*[m.shape[0] for m in matrices]), (ctypes.c_int * n)(*[m.shape[1] for m in matrices]),
+             (ctypes.c_void_p * n)(*[o.data_ptr() for o in out]), nat.stream_of(buf))
+    return out

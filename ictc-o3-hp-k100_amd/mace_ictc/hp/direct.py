@@ -20,7 +20,7 @@ from ictc_o3.ops import tensor_product as tpo
 from ictc_o3.ops.activation import _silu
 from ictc_o3.ops.geometry import _vector_adjoint, edge_harmonics_adjoint_raw, edge_harmonics_raw, shift_vectors
 from ictc_o3.ops.linear import (_fast_ok, _species_apply, degree_layout, packed_linear_adjoint_raw,
-                                packed_linear_raw, path_layout, species_order)
+                                packed_linear_raw, path_layout, species_order, transposed)
 from ictc_o3.ops.radial_mlp import (edge_linear_adjoint_raw, edge_linear_raw, fused_supported,
                                     radial_gates_tangent)
 from ictc_o3.ops.symmetric_contraction import (ICTDBridgeUSymmetricContractionSO3, MaceSymmetricContraction,
@@ -109,28 +109,37 @@ def _species_linear_adjoint(g, weight, species):
     return edge_linear_adjoint_raw(spread.reshape(-1, S * Co), weight.reshape(S * Co, Ci))
 
 
+def _c(w):
+    w = w.detach()
+    return w if w.is_contiguous() else w.contiguous()
+
+
 class _Layer:
-    """One interaction and product: forward() keeps what adjoint() reads."""
+    """One interaction and product: forward() keeps what adjoint() reads.  The weights are read anew on each call
+    (nothing tells of a write through weight.data), and the layer's transposes made in one launch."""
 
     def __init__(self, model, i, species, topo, cfg):
         self.inter, self.prod = model.interactions[i], model.products[i]
         self.C, self.first, self.species, self.topo, self.cfg = model.channels, i == 0, species, topo, cfg
         inter, prod = self.inter, self.prod
         up = inter.linear_up
-        self.up_w = [up.adapters[str(l)].weight.detach() for l in range(up.lmax + 1)]
+        self.up_w = [_c(up.adapters[str(l)].weight) for l in range(up.lmax + 1)]
         self.up_layout = degree_layout(self.up_w, self.C, up.lmax)
         ml = inter.message_linear
-        self.ml_w = [ml.weights[str(l)].detach() for l in range(ml.lmax + 1)]
+        self.ml_w = [_c(ml.weights[str(l)]) for l in range(ml.lmax + 1)]
         self.ml_layout = path_layout(self.ml_w, ml.counts, self.C, ml.lmax, 1.0 / max(inter.avg_num_neighbors, 1e-8))
-        self.pl_w = [w.detach() for w in prod.linear.blocks()]
-        self.pl_layout = degree_layout(self.pl_w, self.C, prod.target_lmax, self.C ** -0.5)
+        self.pl_wt = [_c(w.t()) for w in prod.linear.blocks()]    # the blocks are transposed views of the weight
+        self.pl_layout = degree_layout(self.pl_wt, self.C, prod.target_lmax, self.C ** -0.5)
         self.sc = prod.symmetric_contractions
-        self.sc_w = [w.detach() if w.is_contiguous() else w.detach().contiguous() for w in self.sc.slot_weights()]
+        self.sc_w = [_c(w) for w in self.sc.slot_weights()]
         self.holder = _SpeciesHolder(species, self.sc.num_elements, shared=True)
         self.Ws = [m.weight.detach() for m in inter.fc if isinstance(m, nn.Linear)]
         if model.radial_basis_scale != 1.0:
             self.Ws[0] = self.Ws[0] * model.radial_basis_scale
-        self.Ws = [w if w.is_contiguous() else w.contiguous() for w in self.Ws]
+        self.Ws = [_c(w) for w in self.Ws]
+        made = iter(transposed(self.pl_wt + self.ml_w + ([] if self.first else self.up_w)))
+        self.pl_w, self.ml_wt = [next(made) for _ in self.pl_wt], [next(made) for _ in self.ml_w]
+        self.up_wt = list(made)
 
     def _message(self, h, h0, r, Y, mask, table):
         spec, topo = self.inter.spec(), self.topo
@@ -163,10 +172,10 @@ class _Layer:
     def adjoint(self, dout):
         """Cotangent of the layer's output -> (dh or None, d of its self-connection input or None, dY, dr)."""
         spec, topo = self.inter.spec(), self.topo
-        dcon = packed_linear_adjoint_raw(dout, self.pl_layout, self.pl_w)
+        dcon = packed_linear_adjoint_raw(dout, self.pl_layout, self.pl_wt)
         dmsg = _dx_raw(self.sc.spec(), self.message, self.species, self.sc_w, dcon, holder=self.holder)
         del self.message, dcon
-        go = packed_linear_adjoint_raw(dmsg, self.ml_layout, self.ml_w)
+        go = packed_linear_adjoint_raw(dmsg, self.ml_layout, self.ml_wt)
         del dmsg
         rows, want = topo.gate_rows, not self.first
         if self.form == "species":
@@ -184,7 +193,7 @@ class _Layer:
             return None, None, dY, dr
         ds = dout if dout.shape[1] == self.C else dout[:, :self.C].contiguous()
         ds = _species_linear_adjoint(ds, self.inter.self_connection.weights["0"].detach(), self.species)
-        return packed_linear_adjoint_raw(dx, self.up_layout, self.up_w), ds, dY, dr
+        return packed_linear_adjoint_raw(dx, self.up_layout, self.up_wt), ds, dY, dr
 
 
 @torch.no_grad()

@@ -392,6 +392,11 @@ int ictc_packed_linear(int lmax, int channels_in, int channels_out, const float*
                        const int* out_paths, const int64_t* out_offsets, const float* const* weights,
                        const float* scales, int64_t nodes, void* stream);
 
+/* dst[k] [cols[k], rows[k]] = transpose of src[k] [rows[k], cols[k]], row-major, for k < count in one launch per 64
+ * matrices (host arrays of device pointers; sides up to 2^20): the transposed weights of a call's packed linears. */
+int ictc_transpose(int count, const float* const* src, const int* rows, const int* cols, float* const* dst,
+                   void* stream);
+
 /* ---- Gate projection --------------------------------------------------------
  * Replaces the last Linear of the radial MLP `fc` as the gate projection
  * (layers.py:826-835; streamed_gate_message.py:51-57 `_gate_projection`):

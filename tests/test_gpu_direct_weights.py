@@ -71,3 +71,44 @@ def test_node_embedding(device, monkeypatch, change, S):
     change(w, -0.5 * w.detach())
     moved = rel_err(_check(monkeypatch, model, args, change.__name__), before)
     assert moved > 1e-2
+
+
+WEIGHTS = {"linear_up": lambda m: m.interactions[1].linear_up.adapters["1"].weight,
+           "message_linear": lambda m: m.interactions[1].message_linear.weights["2"],
+           "product": lambda m: m.products[0].linear.weight,
+           "self_connection": lambda m: m.interactions[1].self_connection.weights["0"],
+           "contraction": lambda m: m.products[0].symmetric_contractions.slot_weights()[0],
+           "radial": lambda m: m.interactions[1].fc[2].weight}
+
+
+@pytest.mark.parametrize("change", [_in_place, _through_data, _new_storage])
+@pytest.mark.parametrize("name", WEIGHTS)
+def test_other_weights(device, monkeypatch, change, name):
+    model, args = _model(device, 3), _system(device, 3)
+    w = WEIGHTS[name](model)
+    before = _check(monkeypatch, model, args, "as built")
+    change(w, -0.5 * w.detach() + 0.1)
+    moved = rel_err(_check(monkeypatch, model, args, change.__name__), before)
+    assert moved > 1e-4
+
+
+def test_calls_keep_no_copies_of_weights(device):
+    from ictc_o3.ops import linear
+    from mace_ictc.hp import energy_and_forces
+    model, args = _model(device, 3), _system(device, 3)
+    energy_and_forces(model, *args)
+    linear._operand_cache.clear()
+    torch.cuda.synchronize()
+    held = torch.cuda.memory_allocated()
+    for _ in range(3):
+        energy_and_forces(model, *args)
+    assert not linear._operand_cache and torch.cuda.memory_allocated() == held
+
+
+@pytest.mark.parametrize("shapes", [[(1, 1)], [(33, 31)], [(64, 5), (0, 7), (128, 2176), (32, 32), (5, 0), (1, 200)],
+                                    [(k % 40 + 1, 70 - k) for k in range(65)]])    # 64 matrices a launch
+def test_transposed(device, shapes):
+    from ictc_o3.ops.linear import transposed
+    mats = [torch.randn(*s, device=device) for s in shapes]
+    for m, t in zip(mats, transposed(mats)):
+        assert t.is_contiguous() and t.data_ptr() % 16 == 0 and torch.equal(t, m.t())
