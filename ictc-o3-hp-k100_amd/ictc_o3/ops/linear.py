@@ -240,21 +240,25 @@ _operand_cache = {}   # id(base) -> (weakref to base, {view key: contiguous oper
 def _weight_operand(w, transpose=False):
     """w (or w.t()) detached and contiguous, as the packed kernel reads it.  A non-contiguous view (the
     product linear's transposed blocks) or a transpose (the input adjoint) costs a copy launch; the copy is
-    kept per live base tensor, view geometry and version counter (an optimizer step bumps the version), so
-    a model whose weights do not change between steps makes it once."""
+    kept per live base tensor, view geometry, storage address and version counter (an optimizer step bumps the
+    version) and goes with its base: autograd callers, which hand in the parameter or a view of it, make it once
+    while the weights do not change.  A detached w is a base of its own, so its copy is not found again.  A
+    write through w.data bumps no counter and is not seen."""
     import weakref
     v = w.detach().t() if transpose else w.detach()
     if v.is_contiguous():
         return v
     base = w._base if w._base is not None else w
-    key = (v.storage_offset(), tuple(v.shape), tuple(v.stride()), w._version, v.dtype, v.device)
-    entry = _operand_cache.get(id(base))
+    key = (v.data_ptr(), tuple(v.shape), tuple(v.stride()), w._version, v.dtype, v.device)
+    slot = id(base)
+    entry = _operand_cache.get(slot)
     if entry is None or entry[0]() is not base:
-        if len(_operand_cache) > 256:
-            for k in [k for k, (ref, _) in _operand_cache.items() if ref() is None]:
-                del _operand_cache[k]
-        entry = (weakref.ref(base), {})
-        _operand_cache[id(base)] = entry
+        def drop(ref):
+            held = _operand_cache.get(slot)
+            if held is not None and held[0] is ref:
+                del _operand_cache[slot]
+        entry = (weakref.ref(base, drop), {})
+        _operand_cache[slot] = entry
     views = entry[1]
     out = views.get(key)
     if out is None:

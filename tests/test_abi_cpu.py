@@ -177,6 +177,23 @@ def test_weight_operand_cache_follows_versions():
     assert _weight_operand(c) is not None and _weight_operand(c).data_ptr() == c.data_ptr()
 
 
+def test_weight_operands_go_with_their_base_and_follow_its_storage():
+    """A copy is dropped when its base tensor dies (no dead entry holds memory), and a new storage given to a live
+    base, which leaves its version counter as it was, gives a fresh copy."""
+    from ictc_o3.ops import linear
+    linear._operand_cache.clear()
+    w = torch.nn.Parameter(torch.randn(16, 16))
+    for _ in range(3):      # a detached alias per call, as a backward pass hands in
+        assert torch.equal(linear._weight_operand(w.detach(), transpose=True), w.t())
+    assert not linear._operand_cache
+    assert torch.equal(linear._weight_operand(w, transpose=True), w.t()) and len(linear._operand_cache) == 1
+    version = w._version
+    w.data = torch.randn(16, 16)
+    assert w._version == version and torch.equal(linear._weight_operand(w, transpose=True), w.t())
+    del w
+    assert not linear._operand_cache
+
+
 def test_species_entry_points_host_checks():
     """Argument checks of the species-sorted self connection and its weight gradient (no device work)."""
     from ictc_o3 import _native
