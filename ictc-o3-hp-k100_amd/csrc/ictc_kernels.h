@@ -400,16 +400,17 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kEdgeBwd, T::LI, T::LE, T::LO>::
   load_harmonics<T>(a.sh, e, y);
 #pragma unroll
   for (int j = 0; j < T::NY; ++j) dyv[j] = 0.f;
-  if constexpr (MUL) {   // lanes past the channels hold zero rows: they add nothing to dyv
+  if constexpr (MUL) {   // lanes past the channels hold zero rows and gates: they add nothing to dyv
     __shared__ float turn[kWavesPerBlock][kTurn * kWave];
     float* lds = turn[wave_id()];
     float xv[T::NX], gw[T::P], go[T::NO];
     Turn<FeatureMap<T>, T::NX>::load(a.x + e * (int64_t)(T::NX * C), C, 64 * rg.group, lds, xv);
     Turn<OutputMap<T>, T::NO>::load(grad + e * (int64_t)(T::NO * C), C, 64 * rg.group, lds, go);
     load_gw<T>(a, gate_row(a, e), active ? c : C - 1, 1.f, gw);
-    if (!active) {
+    if (!active) {   // the gates as well: an infinite one times a zero row is NaN
       zero_row<T::NX>(xv);
       zero_row<T::NO>(go);
+      zero_row<T::P>(gw);
     }
     if (dx) {
       float d[T::NX];

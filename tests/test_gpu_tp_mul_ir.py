@@ -56,3 +56,22 @@ def test_mul_ir_rows(device, li, le, lo, C, E):
     for third in (False, True):
         for k, (a, b) in enumerate(zip(run(ops[1], True, third), run(ops[0], False, third))):
             assert rel_err(a, b) < TOL, (third, k)
+
+
+@pytest.mark.parametrize("C", [17, 64, 100])
+def test_infinite_gate_of_the_last_channel(device, C):
+    """An infinite gate of the scalar path: its products are infinite, and no idle lane makes a NaN of them."""
+    from ictc_o3 import EdgeTensorProduct
+    E, grads = 5, []
+    for layout in ("ir_mul", "mul_ir"):
+        op = EdgeTensorProduct.create(input_lmax=1, edge_lmax=1, output_lmax=1, channels=C, layout=layout, device=device)
+        assert op.paths[0] == (0, 0, 0)
+        x = torch.ones(E, 4 * C, device=device)
+        sh = torch.cat(orc.direction_harmonics(unit_vectors(E, 4), 1), -1).float().to(device).requires_grad_(True)
+        gates = torch.ones(E, op.gate_width, device=device)
+        gates[:, C - 1] = float("inf")
+        out = op(x, sh, gates)
+        grads.append(torch.autograd.grad(out, sh, torch.ones_like(out))[0])
+    assert bool(torch.isinf(grads[0][:, 0]).all()) and bool(torch.isfinite(grads[0][:, 1:]).all())
+    # (of the row's finite values: the layouts' sums in another order)
+    assert torch.allclose(grads[1], grads[0], rtol=1e-5, atol=1e-5 * C)
