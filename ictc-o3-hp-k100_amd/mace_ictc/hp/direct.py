@@ -78,7 +78,8 @@ def _plain_context() -> bool:
 
 def _covered(model, pos, A, batch, edge_src, edge_dst, shifts, cell) -> bool:
     tensors = (pos, A, batch, edge_src, edge_dst, shifts, cell)
-    if not (DIRECT and all(type(t) is torch.Tensor and t.is_cuda and not t.requires_grad for t in tensors)
+    if not (DIRECT and pos.is_cuda
+            and all(type(t) is torch.Tensor and t.device == pos.device and not t.requires_grad for t in tensors)
             and pos.dtype == torch.float32 and edge_src.numel() > 0 and model.number_of_basis == 8
             and model.num_elements > 1):      # the packed linear takes no one-row species table
         return False
@@ -90,6 +91,25 @@ def _covered(model, pos, A, batch, edge_src, edge_dst, shifts, cell) -> bool:
                 and all(counts.get(l, 0) > 0 for l in range(inter.lmax + 1))):
             return False
     return all(p.dtype == torch.float32 and p.device == pos.device for p in model.parameters())
+
+
+def _graph_ids(batch, graphs):
+    """Starts reading the range of the graph ids; the function returned raises where one is outside [0, graphs).
+    (The autograd route fails on such an id in the gather of the energies' adjoint, which these sweeps do not have.)
+    Read with the call's first launches and waited for at its end, only that copy: nothing stalls for it."""
+    if graphs == 1 or batch.numel() == 0 or torch.cuda.is_current_stream_capturing():
+        return lambda: None      # one graph: the ids are not used; a captured stream has nothing to read yet
+    host = torch.empty(2, dtype=batch.dtype, pin_memory=True)
+    host.copy_(torch.stack(torch.aminmax(batch)), non_blocking=True)
+    event = torch.cuda.Event()
+    event.record(torch.cuda.current_stream(batch.device))
+
+    def check():
+        event.synchronize()
+        low, high = host.tolist()
+        if low < 0 or high >= graphs:
+            raise ValueError(f"Graph ids run from {low} to {high}, outside 0..{graphs - 1}")
+    return check
 
 
 def _species_linear(x, weight, species):
@@ -205,6 +225,7 @@ def energy_forces(model, pos, A, batch, edge_src, edge_dst, shifts, cell, topolo
         return None
     N, C = pos.shape[0], model.channels
     pos = pos if pos.is_contiguous() else pos.contiguous()
+    check_graph_ids = _graph_ids(batch, cell.shape[0])
     species = model.species_indices(A)
     topo = topology if topology is not None else tpo.Topology(edge_src, edge_dst, N,
                                                               positions=pos if cell.shape[0] == 1 else None)
@@ -254,4 +275,6 @@ def energy_forces(model, pos, A, batch, edge_src, edge_dst, shifts, cell, topolo
         dr, dY = dr + a, dY + b
     rest = cot[-1] if len(cot) > 1 else (None, None)
     dvec = edge_harmonics_adjoint_raw(r, n, (dr, dY, *rest), model.ictd_fix_edge_lmax)
-    return atomic, energy64, -_vector_adjoint(dvec, topo, N)
+    forces = -_vector_adjoint(dvec, topo, N)
+    check_graph_ids()
+    return atomic, energy64, forces
