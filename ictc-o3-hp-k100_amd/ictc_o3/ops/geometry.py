@@ -97,6 +97,14 @@ class _EdgeHarmonics(torch.autograd.Function):
 
 def edge_harmonics_raw(pos, shift, topo, cutoff: float, lmax: int):
     """(r, n, mask, Y) of the edges (no autograd)."""
+    if pos.dtype != torch.float32 or (shift is not None and shift.dtype != torch.float32):
+        raise TypeError("edge_harmonics runs in float32")
+    if pos.dim() != 2 or pos.shape[1] != 3:
+        raise ValueError("pos must be [N, 3]")
+    if shift is not None and tuple(shift.shape) != (topo.src.numel(), 3):
+        raise ValueError("shift must be [E, 3]")
+    if not 0 <= int(lmax) <= 3:
+        raise ValueError("edge_harmonics: lmax outside 0..3")
     pos = _c(pos.detach())
     shift = None if shift is None else _c(shift.detach())
     E, N = topo.src.numel(), pos.shape[0]
@@ -123,14 +131,6 @@ def edge_harmonics(pos: torch.Tensor, shift: torch.Tensor | None, topo, cutoff: 
     """(r [E], Y [E, (lmax+1)^2], mask [E]): edge_geometry followed by the packed direction harmonics of n, in one
     kernel, float32, first derivatives only (positions and shifts).  uses = 2 returns (r, r', Y, Y', mask) with
     r' and Y' the same values for a second consumer, whose cotangents the adjoint adds in its kernel."""
-    if pos.dtype != torch.float32 or (shift is not None and shift.dtype != torch.float32):
-        raise TypeError("edge_harmonics runs in float32")
-    if pos.dim() != 2 or pos.shape[1] != 3:
-        raise ValueError("pos must be [N, 3]")
-    if shift is not None and tuple(shift.shape) != (topo.src.numel(), 3):
-        raise ValueError("shift must be [E, 3]")
-    if not 0 <= int(lmax) <= 3:
-        raise ValueError("edge_harmonics: lmax outside 0..3")
     if uses not in (1, 2):
         raise ValueError("edge_harmonics: uses is 1 or 2")
     return _EdgeHarmonics.apply(pos, shift, topo, float(cutoff), int(lmax), int(uses))

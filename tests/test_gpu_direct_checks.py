@@ -1,5 +1,6 @@
 """energy_and_forces(training=False) without autograd refuses what the autograd route refuses: graph ids outside the
-batch (every kernel that reads them checks them, so nothing is read out of range before the call raises)."""
+batch (every kernel that reads them checks them, so nothing is read out of range before the call raises), and edge
+shifts that are not one per edge (refused on the host before a launch)."""
 import pytest
 import torch
 
@@ -39,3 +40,15 @@ def test_one_graph_ignores_the_ids(device):
     ref = energy_and_forces(model, *args)
     got = energy_and_forces(model, *args[:2], args[2] + 5, *args[3:])
     assert torch.equal(got["forces"], ref["forces"]) and torch.equal(got["energy"], ref["energy"])
+
+
+@pytest.mark.parametrize("paired", [True, False])      # pairing the edges looks at the shifts as well
+@pytest.mark.parametrize("more", [-1, 1])
+def test_shifts_one_per_edge(device, monkeypatch, paired, more):
+    from ictc_o3.ops import tensor_product as tpo
+    from mace_ictc.hp import energy_and_forces
+    model, args = _batch(device, 1)
+    shifts = args[5][:-1] if more < 0 else torch.cat([args[5], args[5][:1]])
+    monkeypatch.setattr(tpo, "PAIR_GATES", paired)
+    with pytest.raises(ValueError, match=r"\[E, 3\]"):
+        energy_and_forces(model, *args[:5], shifts, args[6])
