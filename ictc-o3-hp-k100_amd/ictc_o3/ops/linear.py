@@ -78,12 +78,16 @@ _order_memo = None
 
 
 def species_order(species: torch.Tensor, S: int) -> SpeciesOrder:
-    """SpeciesOrder of this species tensor, kept while the same unmodified tensor is passed again (both
-    layers of a step and their backward share one sort)."""
+    """SpeciesOrder of this species tensor, kept while the same unmodified tensor is passed again on the same
+    stream (both layers of a step and their backward share one sort).  Not kept from or for a captured stream: the
+    order would be read before a replay makes it, or freed while a graph still reads it."""
     global _order_memo
-    key = (species.data_ptr(), species._version, species.shape[0], S, species.device)
-    if _order_memo is not None and _order_memo[0] == key and _order_memo[1] is species:
-        return _order_memo[2]
+    if species.is_cuda and torch.cuda.is_current_stream_capturing():
+        return SpeciesOrder(species, S)
+    key = (species.data_ptr(), species._version, species.shape[0], S, species.device, nat.stream_of(species))
+    memo = _order_memo      # read once: another thread may replace it between two reads
+    if memo is not None and memo[0] == key and memo[1] is species:
+        return memo[2]
     order = SpeciesOrder(species, S)
     _order_memo = (key, species, order)
     return order
