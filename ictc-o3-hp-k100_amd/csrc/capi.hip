@@ -533,13 +533,20 @@ int ictc_tp_bwd_mul_ir(int li, int le, int lo, int C, const float* x, const floa
   return tp_bwd(li, le, lo, C, x, sh, g, w, grad, E, dx, dsh, dg, workspace, workspace_bytes, true, stream);
 }
 
+// What ictc_csr_build needs for this list: the counting sort's or the library sort's storage.
+static int64_t counting_bytes(int64_t E) {
+  return (int64_t)(count_bytes(E > 0 ? (E + kTile - 1) / kTile : 1) + align256(3 * sizeof(int32_t) * (size_t)(E > 0 ? E : 1)));
+}
+static int64_t csr_bytes(int64_t E, int64_t N) {
+  if (sort_passes(E, N)) return counting_bytes(E);
+  return (int64_t)(3 * align256(sizeof(int32_t) * (size_t)(E > 0 ? E : 1)) + align256(sort_temp_bytes(E, N)));
+}
+
 int64_t ictc_csr_workspace_bytes(int64_t E, int64_t N) {
   if (E < 0 || N < 0 || E >= (int64_t(1) << 31) || N >= (int64_t(1) << 31) - 2) return -1;
-  if (sort_passes(E, N)) {
-    const size_t tiles = (size_t)(E > 0 ? (E + kTile - 1) / kTile : 1);
-    return (int64_t)(count_bytes((int64_t)tiles) + align256(3 * sizeof(int32_t) * (size_t)(E > 0 ? E : 1)));
-  }
-  return (int64_t)(3 * align256(sizeof(int32_t) * (size_t)(E > 0 ? E : 1)) + align256(sort_temp_bytes(E, N)));
+  // A workspace made for the largest list serves every smaller one: past the counting sort's range the answer
+  // covers it too (its counts take more than the library sort near the range's end).
+  return std::max(csr_bytes(E, N), counting_bytes(std::min(E, kSmallSort)));
 }
 
 int ictc_csr_build(const int64_t* keys, int64_t E, int64_t N, int32_t* ptr, int32_t* order, void* workspace,
@@ -560,7 +567,7 @@ int ictc_csr_build(const int64_t* keys, int64_t E, int64_t N, int32_t* ptr, int3
     return check_hip(hipGetLastError(), "csr ptr (sorted keys)");
   }
   if (!workspace) return fail(ICTC_ERR_ARGUMENT, "csr: null workspace");
-  const int64_t need = ictc_csr_workspace_bytes(E, N);
+  const int64_t need = csr_bytes(E, N);
   if (workspace_bytes < need)
     return fail(ICTC_ERR_ARGUMENT, "csr: workspace of %lld bytes, need %lld", (long long)workspace_bytes,
                 (long long)need);

@@ -104,7 +104,8 @@ int ictc_tp_second(int input_lmax, int edge_lmax, int output_lmax, int channels,
  *   ptr   [nodes + 2] int32: edges of node n are order[ptr[n] .. ptr[n+1]);
  *         ptr[nodes] .. ptr[nodes+1] holds edges whose key is out of range;
  *   order [E] int32, a stable sort of edge ids by key.
- * workspace must hold ictc_csr_workspace_bytes(edges, nodes) bytes.  order
+ * workspace must hold ictc_csr_workspace_bytes(edges, nodes) bytes (enough for
+ * every list of at most that many edges and nodes).  order
  * NULL: the caller guarantees keys already in non-decreasing order with every
  * key in [0, nodes) (a receiver-sorted edge list, e.g. the neighbour list's);
  * only ptr is built, the order is the identity (pass NULL as dst_order), and

@@ -194,6 +194,18 @@ def test_weight_operands_go_with_their_base_and_follow_its_storage():
     assert not linear._operand_cache
 
 
+def test_csr_workspace_covers_smaller_lists():
+    """A workspace made for the largest list of a run serves every smaller one (the library sort's temporary storage
+    is known only on a device, so this is the part that the list itself takes)."""
+    from ictc_o3 import _native
+    f = _native.lib().ictc_csr_workspace_bytes
+    edges = (0, 1, 1000, 1024, 1025, 100000, 262143, 262144, 262145, 270000, 300000, 10 ** 6)
+    nodes = (0, 255, 256, 65535, 65536, 10 ** 6)
+    size = [[f(E, N) for N in nodes] for E in edges]
+    assert all(a <= b for row in size for a, b in zip(row, row[1:]))
+    assert all(a <= b for r, s in zip(size, size[1:]) for a, b in zip(r, s))
+
+
 def test_species_entry_points_host_checks():
     """Argument checks of the species-sorted self connection and its weight gradient (no device work)."""
     from ictc_o3 import _native

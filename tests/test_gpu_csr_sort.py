@@ -20,3 +20,18 @@ def test_csr_is_a_stable_sort(device, E, N):
     assert torch.equal(csr.order[:E].long().cpu(), torch.argsort(k, stable=True))
     want = torch.cat([torch.searchsorted(k.sort().values, torch.arange(N + 1)), torch.tensor([E])])
     assert torch.equal(csr.ptr.long().cpu(), want)
+
+
+@pytest.mark.parametrize("largest,E,N", [((262145, 4096), 262144, 4096), ((262145, 4096), 1000, 100),
+                                         ((1000, 65536), 1000, 4096), ((1000, 65536), 1000, 100),
+                                         ((1000, 65536), 1, 65536)])
+def test_workspace_of_a_larger_list(device, largest, E, N):
+    from ictc_o3 import _native as nat
+    nbytes = int(nat.lib().ictc_csr_workspace_bytes(*largest))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    keys = torch.randint(0, N, (E,), device=device, generator=torch.Generator(device=device).manual_seed(E))
+    ptr = torch.empty(N + 2, dtype=torch.int32, device=device)
+    order = torch.empty(E, dtype=torch.int32, device=device)
+    nat.call("ictc_csr_build", nat.ptr(keys), E, N, nat.ptr(ptr), nat.ptr(order), nat.ptr(ws), nbytes,
+             nat.stream_of(keys))
+    assert torch.equal(order.long(), torch.argsort(keys, stable=True))
