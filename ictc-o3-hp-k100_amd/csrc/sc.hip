@@ -207,7 +207,7 @@ int check_tab(int li, int lt, int corr, int C, int S, int64_t N, int dw, Shape* 
                 li, lt, corr);
   if (S > 65535) return fail(ICTC_ERR_UNSUPPORTED, "symmetric contraction table: more than 65535 species");
   if (N >= (int64_t(1) << 31)) return fail(ICTC_ERR_UNSUPPORTED, "symmetric contraction table: more than 2^31 nodes");
-  *floats = dw ? (ictc::sc::tab_max_chunks(N, pairs, C, S) + S) * pairs * C : ictc::sc::tab_floats(pairs, C, S);
+  *floats = dw ? ictc::sc::tab_max_chunks(N, pairs, C, S) * pairs * C : ictc::sc::tab_floats(pairs, C, S);
   return ICTC_OK;
 }
 

@@ -79,16 +79,24 @@ def term_count(spec) -> int:
 # group) waves the per-node kernels are as fast (one wave per node fills more of the GPU): lmax 3 over 2,048
 # nodes of 64 channels 54 -> 36 us forward but 17 us for the order; lmax 2, whose terms outnumber its pairs less,
 # 18 -> 19 us over 8,000 nodes and 266 -> 190 over 131,072 (its weight gradients, which take the order anyway,
-# 85 -> 68 and 1,390 -> 515).  With few nodes per species the table costs what it saves.
+# 85 -> 68 and 1,390 -> 515).
 _TABLE_WAVES = {3: 4096, 2: 32768}
 _TABLE_WEIGHT_WAVES = 4096
-_TABLE_NODES_PER_SPECIES = 32
+# The table, and the weight gradient's pair sums, grow with the species: with few nodes of each they cost what they
+# save.  Per-node -> table, us: (3,1), 8,191 nodes of 64 channels, 48 a species: forward 76 -> 73, feature gradient
+# 96 -> 80, weight gradient 112 -> 96; 32: 77 -> 96, 98 -> 105, 137 -> 110.  (3,2), 32,768 nodes of 64 channels, 64:
+# 855 -> 522, 1,060 -> 600, 726 -> 704; 48: 859 -> 643, 1,064 -> 712, 745 -> 905.  (2,2), 131,072 nodes, 256: 261 ->
+# 250, 338 -> 296, 431 -> 392; 128: 314 -> 317, 359 -> 372, 467 -> 402; 96: 329 -> 368, 367 -> 427, 499 -> 559.
+_TABLE_NODES_PER_SPECIES = {3: 64, 2: 256}
+_TABLE_WEIGHT_NODES_PER_SPECIES = {3: 64, 2: 128}
 
 
 def _use_table(spec, N, weights=False) -> bool:
+    if spec.pairs == 0 or not 0 < spec.num_species <= 65535 or N >= 2 ** 31:   # (what the table kernels take)
+        return False
     waves = N * ((spec.channels + 63) // 64)
-    return (spec.pairs > 0 and waves >= (_TABLE_WEIGHT_WAVES if weights else _TABLE_WAVES[spec.lmax])
-            and N >= _TABLE_NODES_PER_SPECIES * spec.num_species)
+    per = (_TABLE_WEIGHT_NODES_PER_SPECIES if weights else _TABLE_NODES_PER_SPECIES)[spec.lmax]
+    return waves >= (_TABLE_WEIGHT_WAVES if weights else _TABLE_WAVES[spec.lmax]) and N >= per * spec.num_species
 
 
 def _table_raw(spec, x, csr, ws, go=None, tangent=None):

@@ -16,7 +16,9 @@ TOL = 1e-5
 
 
 @pytest.mark.parametrize("lmax,lt,C,N,S", [(2, 2, 64, 1, 1), (2, 2, 70, 333, 3), (3, 1, 17, 47, 2), (3, 1, 64, 129, 1),
-                                           (3, 2, 64, 16, 2), (3, 2, 100, 2100, 7)])
+                                           (3, 2, 64, 16, 2), (3, 2, 100, 2100, 7),
+                                           # 64 species a step of the tile search: its edges, and more nodes than one tile
+                                           (2, 2, 64, 900, 63), (3, 1, 64, 500, 64), (2, 2, 16, 3000, 200)])
 def test_table_kernels_match_per_node(device, lmax, lt, C, N, S, monkeypatch):
     from ictc_o3.ops import symmetric_contraction as sco
     mod, x64, species = _setup(device, lmax, lt, 3, C, N, S, 5)
