@@ -208,11 +208,13 @@ __device__ __forceinline__ void load_gw(const Operands& a, int64_t row, int c, f
 // ---------------------------------------------------------------------------
 constexpr int kMaxGroups = 4;
 
-// Minimum waves per SIMD requested for each (kernel, degree triple): the
-// highest of 4, 3, 2, 1 at which the kernel compiles without register spills,
-// found by tune_occupancy.py and recorded in ictc_occupancy.h.
+// Minimum waves per SIMD requested for each (kernel instance, degree triple):
+// the highest of 4, 3, 2, 1 at which it compiles with at most 8 spilled VGPRs
+// (three measured exceptions), found by tune_occupancy.py and recorded in
+// ictc_occupancy.h.
 enum KernelKind {
-  kEdgeFwd, kEdgeBwd, kMsgFwd, kMsgBwdEdge, kMsgBwdX, kEdgeSecond, kMsgFwd2, kMsgBwdEdge2, kMsgBwdX2
+  kEdgeFwd, kEdgeFwdMul, kEdgeBwd, kEdgeBwdMul, kMsgFwd, kMsgBwdEdge, kMsgBwdX, kEdgeSecond, kMsgFwd2, kMsgFwd2All,
+  kMsgBwdEdge2, kMsgBwdX2, kMsgBwdX2All
 };
 template <int K, int LI, int LE, int LO>
 struct Occupancy {
@@ -360,7 +362,7 @@ struct OutputMap {
 // Edge TP: one wave per (edge, channel group).  MUL: features, output and their gradients are mul_ir rows.
 // ---------------------------------------------------------------------------
 template <class T, bool MUL>
-__global__ __launch_bounds__(kBlock, (Occupancy<kEdgeFwd, T::LI, T::LE, T::LO>::value)) void edge_fwd_kernel(
+__global__ __launch_bounds__(kBlock, (Occupancy<MUL ? kEdgeFwdMul : kEdgeFwd, T::LI, T::LE, T::LO>::value)) void edge_fwd_kernel(
     Operands a, float* __restrict__ out) {
   const RowGroup rg = row_group_y();
   const int64_t e = rg.row;
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kEdgeFwd, T::LI, T::LE, T::LO>::
 }
 
 template <class T, bool MUL>
-__global__ __launch_bounds__(kBlock, (Occupancy<kEdgeBwd, T::LI, T::LE, T::LO>::value)) void edge_bwd_kernel(
+__global__ __launch_bounds__(kBlock, (Occupancy<MUL ? kEdgeBwdMul : kEdgeBwd, T::LI, T::LE, T::LO>::value)) void edge_bwd_kernel(
     Operands a, const float* __restrict__ grad, float* __restrict__ dx, float* __restrict__ dsh,
     float* __restrict__ dsh_part, float* __restrict__ dgates) {
   const RowGroup rg = row_group_y();
@@ -934,8 +936,9 @@ struct RollingEdge {
   __device__ __forceinline__ void used_out(int k) { go[k] = row_load<kCached>(next_go, off, k * pitch); }
 };
 
-// Waves per SIMD of the source-owned adjoint: what the edge's values and the row sums leave room for without spills
-// of the unweighted form ((1,3,3) with kTangent, 60 edge values, spills 25 at 4).
+// Waves per SIMD of the source-owned adjoint: what the edge's values and the row sums leave room for ((1,3,3) with
+// kTangent, 60 edge values, spills 25 at 4).  Spilled VGPRs at these counts: none without path weights but 2 at (2,3,1)
+// kTangent and (2,3,2) kAddGrad; with them 3 to 5 at (2,3,2), and 30 (kAddGrad) and 34 (kTangent) at (3,3,3).
 template <class T, GateGrad GRAD, bool W>
 constexpr int src_adjoint_waves() {
   constexpr int edge = T::NO + (1 + RollingEdge<T, GRAD, W>::kTwo + W) * T::P, live = edge + 3 * T::NX + T::NY;

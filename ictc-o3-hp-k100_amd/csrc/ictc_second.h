@@ -146,15 +146,8 @@ __device__ __forceinline__ void stage_tangent(const float* __restrict__ tsh, con
 // first layer), one body that forms the products of x once for both of its terms
 // ((2,3,3) C128 over 424 k edges, VALU-bound: 2,860 -> 2,471 us).
 // ---------------------------------------------------------------------------
-// Waves per SIMD: the one-body form holds both gate rows and both feature rows at once, so the triples that the
-// table gives 4 waves and that have 35 or more outputs ((2,2,2): 133 VGPRs) run at 3.
 template <class T, bool ALL>
-constexpr int fwd2_waves() {
-  constexpr int w = Occupancy<kMsgFwd2, T::LI, T::LE, T::LO>::value;
-  return ALL && w == 4 && T::NO >= 35 ? 3 : w;
-}
-template <class T, bool ALL>
-__global__ __launch_bounds__(kBlock, (fwd2_waves<T, ALL>())) void msg_fwd2_kernel(
+__global__ __launch_bounds__(kBlock, (Occupancy<ALL ? kMsgFwd2All : kMsgFwd2, T::LI, T::LE, T::LO>::value)) void msg_fwd2_kernel(
     Operands a, Tangents t, const int64_t* __restrict__ src, Csr csr, float* __restrict__ out, int parts) {
   const RowGroup rg = row_group_y_xcd();
   const RowShare rs = row_share(csr, rg.row, a.rows, a.rows, parts);
@@ -297,7 +290,7 @@ __global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdEdge2, T::LI, T::LE, T::L
 // Source-owned: dx[s] = sum over edges out of s of dx(ty, g, go) + dx(y, tg, go).  ALL: both tangents are given,
 // and the contraction with go is formed once for both terms ((2,3,3) C128 over 424 k edges: 2,185 -> 1,814 us).
 template <class T, bool ALL>
-__global__ __launch_bounds__(kBlock, (Occupancy<kMsgBwdX2, T::LI, T::LE, T::LO>::value)) void msg_bwd_x2_kernel(
+__global__ __launch_bounds__(kBlock, (Occupancy<ALL ? kMsgBwdX2All : kMsgBwdX2, T::LI, T::LE, T::LO>::value)) void msg_bwd_x2_kernel(
     Operands a, Tangents t, const int64_t* __restrict__ dst, Csr scsr, const float* __restrict__ grad,
     float* __restrict__ dx, int parts) {
   const RowGroup rg = row_group_y_xcd();
