@@ -7,17 +7,18 @@ native_jit.py:17-62); this build instead emits every qualified shape
 (input, edge and output degree <= 3, natural-parity paths) ahead of time, so
 there is no cold-start compiler in the product.
 
-For each (LI, LE, LO) the header defines ``Tp<LI,LE,LO>`` with four device
+For each (LI, LE, LO) the header defines ``Tp<LI,LE,LO>`` with device
 functions operating on per-lane register arrays, indices in the packed
 component order (component k of degree l sits at l*l + m):
 
   fwd   o[k]  += gw[p] * sum C_p[m1,m2,m3] x[m1] y[m2]      (o index: output slot)
-  dx    dx[i] += sum_p gw[p] sum C_p y[m2] go[k]
+  dx_v  dx[i] += sum_p gw[p] sum C_p y[m2] go[k], factorised through V_p[i][j] = sum_k C go[k]
   dy    dy[j] += sum_p gw[p] sum C_p x[m1] go[k]
   dg    dg[p]  = sum_k go[k] sum C_p x[m1] y[m2]
   dydg  dy and dg of the same x in one pass
-  adjoint  dx, dy and dg path by path, factorised through V_p[i][j] = sum_k C go[k]
-  dx_v     the same factorisation for dx alone
+  dydgt  dy and the dot of dg with a tangent row, path by path
+  fwd3_f, dx2_v  the forward and feature-gradient terms of the mixed second derivative together
+  adjoint  dx, dy and dg path by path through the same V_p
 
 The sums are grouped so that the lane-varying operand meets the CG literal
 first: B_jk = sum_i C x[i] costs one VALU op per nonzero, and the per-edge
@@ -93,20 +94,6 @@ def tp_struct(li, le, lo):
                  " const float* __restrict__ gw, float* __restrict__ o) {")
     for k, js in sorted(by_kj.items()):
         lines.append(f"    o[{k}] = fmaf(gw[{path_of[k]}], {t_expr('x', 'y', js)}, o[{k}]);")
-    lines.append("  }")
-    # dx: d[i] += sum_j y[j] sum_p gw[p] sum_{k in p} C go[k]
-    lines.append("  __device__ __forceinline__ static void dx(const float* __restrict__ y, const float* __restrict__ gw,"
-                 " const float* __restrict__ go, float* __restrict__ d) {")
-    by_ij = {}
-    for p, i, j, k, v in ent:
-        by_ij.setdefault(i, {}).setdefault(j, {}).setdefault(p, []).append((k, v))
-    for i, js in sorted(by_ij.items()):
-        parts = []
-        for j, ps in sorted(js.items()):
-            inner = " + ".join(f"gw[{p}] * ({' + '.join(f'{f(v)} * go[{k}]' for k, v in ks)})"
-                               for p, ks in sorted(ps.items()))
-            parts.append(f"y[{j}] * ({inner})")
-        lines.append(f"    d[{i}] += {' + '.join(parts)};")
     lines.append("  }")
     # dy: d[j] += sum_k (gw[p] go[k]) B_jk(x)
     lines.append("  __device__ __forceinline__ static void dy(const float* __restrict__ x, const float* __restrict__ gw,"

@@ -124,21 +124,9 @@ __device__ __forceinline__ void load_row(const float* __restrict__ base, int C, 
   }
 }
 
-// load_row for a row read once: non-temporal loads, so that the streamed row does not displace
-// the rows other waves gather again (the receiver cotangent rows of the source-owned adjoint).
-template <int N>
-__device__ __forceinline__ void load_row_stream(const float* __restrict__ base, int C, int c, float* v) {
-  uint32_t off = (uint32_t)c * 4u;
-  asm volatile("" : "+v"(off));
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    v[i] = __builtin_nontemporal_load(reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off));
-    base += C;
-  }
-}
-
 // A row as a buffer descriptor (wave-uniform base, `bytes` readable) and one component of it: the lane's byte
-// offset in a VGPR, the component's in an SGPR.  kStream: a row read once, as in load_row_stream.
+// offset in a VGPR, the component's in an SGPR.  kStream: a row read once, by non-temporal loads, so that it does not
+// displace the rows other waves gather again (the receiver cotangent rows of the source-owned adjoint).
 constexpr int kCached = 0, kStream = 2;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float* base, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000);
@@ -180,10 +168,9 @@ __device__ __forceinline__ void store_dg_row(const Operands& a, float* __restric
 // Gates of gate row `row` for channel c, times the per-path weight (if any) and `scale`.
 // All P gate loads are issued before any use so they are in flight together;
 // the optional weight is a separate uniform branch after them.
-template <class T, bool STREAM = false>
+template <class T>
 __device__ __forceinline__ void load_gw(const Operands& a, int64_t row, int c, float scale, float* gw) {
-  if (STREAM) load_row_stream<T::P>(a.gates + row * (int64_t)(T::P * a.channels), a.channels, c, gw);
-  else load_row<T::P>(a.gates + row * (int64_t)(T::P * a.channels), a.channels, c, gw);
+  load_row<T::P>(a.gates + row * (int64_t)(T::P * a.channels), a.channels, c, gw);
   if (a.weight) {
     float w[T::P];
 #pragma unroll
