@@ -1,5 +1,5 @@
-"""energy_and_forces(training=False) without autograd refuses what the autograd route refuses: graph ids outside the
-batch (every kernel that reads them checks them, so nothing is read out of range before the call raises), and edge
+"""energy_and_forces(training=False) without autograd at the widest degree, and what it refuses as the autograd route
+does: graph ids outside the batch (every kernel that reads them checks them, so nothing is read out of range before the call raises), and edge
 shifts that are not one per edge (refused on the host before a launch)."""
 import pytest
 import torch
@@ -52,3 +52,21 @@ def test_shifts_one_per_edge(device, monkeypatch, paired, more):
     monkeypatch.setattr(tpo, "PAIR_GATES", paired)
     with pytest.raises(ValueError, match=r"\[E, 3\]"):
         energy_and_forces(model, *args[:5], shifts, args[6])
+
+
+@pytest.mark.parametrize("S", [3, 5])      # the first layer's message: gates materialised (no species form at edge degree 3)
+def test_widest_degree_matches_autograd(device, monkeypatch, S):
+    """lmax 3 and one layer (the contraction onto degree 3, which more layers need, is not compiled)."""
+    from helpers import rel_err
+    from mace_ictc.hp import create_model, direct, energy_and_forces
+    torch.manual_seed(5)
+    zs = (1, 6, 7, 8, 9)[:S]
+    model = create_model(lmax=3, num_interactions=1, atomic_numbers=zs, cutoff=4.5, device=device)
+    pos, Z, batch, cell = fcc_cells(3, 0.1, 0.3, 3, S, cells=1, atomic_numbers=zs)
+    src, dst, sh = build_graph(pos, batch, cell, 4.5)
+    args = [t.to(device) for t in (pos.float(), Z, batch, src, dst, sh.float(), cell.float())]
+    got = energy_and_forces(model, *args)
+    monkeypatch.setattr(direct, "DIRECT", False)
+    ref = energy_and_forces(model, *args)
+    for k in ("energy", "forces", "atomic_energy"):   # two routes of the same kernels: sums in another order
+        assert rel_err(got[k], ref[k]) < 2e-6, k
