@@ -125,11 +125,17 @@ __device__ __forceinline__ void load_row(const float* __restrict__ base, int C, 
 }
 
 // A row as a buffer descriptor (wave-uniform base, `bytes` readable) and one component of it: the lane's byte
-// offset in a VGPR, the component's in an SGPR.  kStream: a row read once, by non-temporal loads, so that it does not
+// offset in a VGPR, the component's in an SGPR.  Read from the first lane here, and the pitch below: where the compiler
+// forms a descriptor or an offset in VGPRs (input degree 1 did), it wraps every access in a loop over the lanes'
+// values (gate-tangent adjoint over 16,384 rows, about 630 k edges of 32 channels: (1,2,2) 571 us, 359 without; (1,3,3)
+// 1,176 and 622).  kStream: a row read once, by non-temporal loads, so that it does not
 // displace the rows other waves gather again (the receiver cotangent rows of the source-owned adjoint).
 constexpr int kCached = 0, kStream = 2;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const float* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000);
+  const uint64_t at = (uint64_t)base;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)at), hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((float*)((uint64_t)hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(bytes),
+                                           0x00027000);
 }
 template <int AUX>
 __device__ __forceinline__ float row_load(__amdgpu_buffer_rsrc_t row, int off, int component) {
@@ -971,6 +977,9 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, GRAD, W>())) void msg
       if constexpr (GRAD == kTangent) ed.next_gt = row_rsrc(gdot + row * (int64_t)(T::P * C), T::P * live);
       if constexpr (GRAD == kAddGrad)
         ed.next_gt = row_rsrc(dgates + lane_i(ch.e, j) * (int64_t)(T::P * C), T::P * live);
+      // Component offsets are formed at their loads: kept across edges they take up to 120 SGPRs, spilled to VGPRs.
+      ed.pitch = __builtin_amdgcn_readfirstlane(C * 4);
+      asm volatile("" : "+s"(ed.pitch));
     };
     point(0);
     if (active) {
@@ -982,9 +991,6 @@ __global__ __launch_bounds__(kBlock, (src_adjoint_waves<T, GRAD, W>())) void msg
     for (int i = 0; i < count; ++i) {
       const int64_t e = lane_i(ch.e, i);
       point(i + 1);
-      ed.pitch = __builtin_amdgcn_readfirstlane(C * 4);
-      // Component offsets are formed at their loads: kept across edges they take up to 120 SGPRs, spilled to VGPRs.
-      asm volatile("" : "+s"(ed.pitch));
       ed.mask = lane_f(ch.m, i);
       if constexpr (GRAD == kTangent) ed.dgt = 0.f;
       else if constexpr (GRAD != kNoGrad) ed.dgates = row_rsrc(dgates + e * (int64_t)(T::P * C), T::P * C * 4);
