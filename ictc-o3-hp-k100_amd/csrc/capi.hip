@@ -159,7 +159,7 @@ size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 // earlier keys (ballots of equal digits), so equal digits keep their order.  Up to 255 distinct keys (species
 // ids) one pass sorts and its scan yields ptr; receiver lists of up to 65,535 rows take two.  Measured (us of
 // kernels): 65,000 edges over 1,359 receivers 65 -> 40 and 10 launches -> 7; 8,191 species ids 37 -> 15 and
-// 8 -> 3.
+// 8 -> 3 (the lists it is used for: prefer_counting).
 constexpr int kDigits = 256, kTile = 1024, kSortWaves = 4, kRounds = kTile / (64 * kSortWaves);
 
 // Lanes of the wave with this lane's digit (all 64 lanes call it; an inactive lane passes active = false).
@@ -296,12 +296,20 @@ __global__ __launch_bounds__(256) void sort_scatter_kernel(const int64_t* __rest
 // Bytes of a pass's counts: whole groups of four for every thread of the scan.
 size_t count_bytes(int64_t tiles) { return sizeof(int32_t) * 4096 * (size_t)((kDigits * tiles + 4095) / 4096); }
 
-// Passes of the counting sort, or 0 where the library sort is used: more than 2^16 keys would need a third
-// pass, and the one-block scan of [256][tiles] grows with the list.
+// Lists the counting sort takes: more than 2^16 keys would need a third pass, and the one-block scan of [256][tiles]
+// grows with the list.
 constexpr int64_t kSmallSort = int64_t(1) << 18;
-int sort_passes(int64_t E, int64_t N) {
-  if (E > kSmallSort || N >= (int64_t(1) << 16)) return 0;
-  return N < kDigits ? 1 : 2;
+bool countable(int64_t E, int64_t N) { return E <= kSmallSort && N < (int64_t(1) << 16); }
+
+// Whether it is the faster one there (us, library -> counting sort).  One pass: always (1,000 keys 15 -> 14).  Two
+// passes: above 4,096 edges, which the library sorts in one or two launches (1,024: 15 -> 24, 4,096: 20 -> 27, 5,000:
+// 29 -> 27); above 200,000, where the library takes its long way (202,000 edges of 65,535 rows 98 -> 84); between them
+// while the second pass's counts are few (131,072 edges of 40,000 rows, 20,096 counts, 58 -> 52; 165,000 of 50,000,
+// 31,752 counts, 64 -> 68; 200,000 of 65,535, 50,176 counts, 67 -> 84).
+bool prefer_counting(int64_t E, int64_t N) {
+  if (!countable(E, N)) return false;
+  if (N < kDigits) return true;
+  return E > 4096 && (E > 200000 || ((N >> 8) + 1) * ((E + kTile - 1) / kTile) <= 24576);
 }
 
 // ---- Spatial (Morton) row order -------------------------------------------
@@ -533,20 +541,20 @@ int ictc_tp_bwd_mul_ir(int li, int le, int lo, int C, const float* x, const floa
   return tp_bwd(li, le, lo, C, x, sh, g, w, grad, E, dx, dsh, dg, workspace, workspace_bytes, true, stream);
 }
 
-// What ictc_csr_build needs for this list: the counting sort's or the library sort's storage.
+// What the two sorts need.
 static int64_t counting_bytes(int64_t E) {
   return (int64_t)(count_bytes(E > 0 ? (E + kTile - 1) / kTile : 1) + align256(3 * sizeof(int32_t) * (size_t)(E > 0 ? E : 1)));
 }
-static int64_t csr_bytes(int64_t E, int64_t N) {
-  if (sort_passes(E, N)) return counting_bytes(E);
+static int64_t library_bytes(int64_t E, int64_t N) {
   return (int64_t)(3 * align256(sizeof(int32_t) * (size_t)(E > 0 ? E : 1)) + align256(sort_temp_bytes(E, N)));
 }
 
 int64_t ictc_csr_workspace_bytes(int64_t E, int64_t N) {
   if (E < 0 || N < 0 || E >= (int64_t(1) << 31) || N >= (int64_t(1) << 31) - 2) return -1;
-  // A workspace made for the largest list serves every smaller one: past the counting sort's range the answer
-  // covers it too (its counts take more than the library sort near the range's end).
-  return std::max(csr_bytes(E, N), counting_bytes(std::min(E, kSmallSort)));
+  // A workspace made for the largest list serves every smaller one: it holds the counting sort of all that take it
+  // (ictc_csr_build falls back to it), and past those the library's.
+  const int64_t counting = counting_bytes(std::min(E, kSmallSort));
+  return prefer_counting(E, N) ? counting : std::max(counting, library_bytes(E, N));
 }
 
 int ictc_csr_build(const int64_t* keys, int64_t E, int64_t N, int32_t* ptr, int32_t* order, void* workspace,
@@ -567,19 +575,22 @@ int ictc_csr_build(const int64_t* keys, int64_t E, int64_t N, int32_t* ptr, int3
     return check_hip(hipGetLastError(), "csr ptr (sorted keys)");
   }
   if (!workspace) return fail(ICTC_ERR_ARGUMENT, "csr: null workspace");
-  const int64_t need = csr_bytes(E, N);
+  // the faster sort, or the other where only that fits the workspace (both are stable: the same order)
+  bool counting = prefer_counting(E, N);
+  if (countable(E, N) && workspace_bytes < (counting ? counting_bytes(E) : library_bytes(E, N))) counting = !counting;
+  const int64_t need = counting ? counting_bytes(E) : library_bytes(E, N);
   if (workspace_bytes < need)
     return fail(ICTC_ERR_ARGUMENT, "csr: workspace of %lld bytes, need %lld", (long long)workspace_bytes,
                 (long long)need);
   char* ws = (char*)workspace;
-  if (const int passes = sort_passes(E, N)) {
+  if (counting) {
     const int64_t tiles = (E + kTile - 1) / kTile;
     int32_t* counts = (int32_t*)ws;
     int32_t* k1 = (int32_t*)(ws + count_bytes(tiles));
     int32_t* id1 = k1 + E;
     int32_t* k2 = id1 + E;
     const dim3 grid((unsigned)tiles), block(256);
-    const bool two = passes == 2;
+    const bool two = N >= kDigits;
     const int d0 = two ? kDigits : (int)N + 1, d1 = (int)(N >> 8) + 1;
     hipLaunchKernelGGL(sort_count_kernel, grid, block, 0, st, keys, (const int32_t*)nullptr, E, N, 0, d0, counts);
     hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(1024), 0, st, counts, d0, (int)tiles, E,

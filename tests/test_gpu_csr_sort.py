@@ -24,7 +24,8 @@ def test_csr_is_a_stable_sort(device, E, N):
 
 @pytest.mark.parametrize("largest,E,N", [((262145, 4096), 262144, 4096), ((262145, 4096), 1000, 100),
                                          ((1000, 65536), 1000, 4096), ((1000, 65536), 1000, 100),
-                                         ((1000, 65536), 1, 65536)])
+                                         ((1000, 65536), 1, 65536), ((5000, 4096), 4096, 4096),
+                                         ((200001, 65535), 200000, 65535)])
 def test_workspace_of_a_larger_list(device, largest, E, N):
     from ictc_o3 import _native as nat
     nbytes = int(nat.lib().ictc_csr_workspace_bytes(*largest))
@@ -35,3 +36,24 @@ def test_workspace_of_a_larger_list(device, largest, E, N):
     nat.call("ictc_csr_build", nat.ptr(keys), E, N, nat.ptr(ptr), nat.ptr(order), nat.ptr(ws), nbytes,
              nat.stream_of(keys))
     assert torch.equal(order.long(), torch.argsort(keys, stable=True))
+
+
+def _bytes(E):
+    """The counting sort's storage (its counts in whole groups of 4,096, keys and ids of both passes)."""
+    tiles = (E + 1023) // 1024
+    return 4 * 4096 * ((256 * tiles + 4095) // 4096) + (12 * E + 255) // 256 * 256
+
+
+@pytest.mark.parametrize("E,N", [(4096, 300), (4097, 300), (1, 256), (200000, 65535), (200001, 65535), (170000, 40000)])
+def test_either_sort_gives_the_stable_order(device, E, N):
+    """On both sides of the rule that chooses the sort; and with room for the counting sort alone, which it then is."""
+    from ictc_o3 import _native as nat
+    keys = torch.randint(0, N, (E,), device=device, generator=torch.Generator(device=device).manual_seed(E))
+    want = torch.argsort(keys, stable=True)
+    for nbytes in (int(nat.lib().ictc_csr_workspace_bytes(E, N)), _bytes(E)):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        ptr = torch.empty(N + 2, dtype=torch.int32, device=device)
+        order = torch.empty(E, dtype=torch.int32, device=device)
+        nat.call("ictc_csr_build", nat.ptr(keys), E, N, nat.ptr(ptr), nat.ptr(order), nat.ptr(ws), nbytes,
+                 nat.stream_of(keys))
+        assert torch.equal(order.long(), want)
