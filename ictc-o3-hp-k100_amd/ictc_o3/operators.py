@@ -171,7 +171,8 @@ class EdgeTensorProduct(torch.nn.Module):
         return result
 
     def forward(self, features, harmonics, gates):
-        """features [E,C*(L_in+1)^2], harmonics [E,(L_edge+1)^2], gates [E,P*C] or [E,P,C] (operators.py:310-340)."""
+        """features [E,C*(L_in+1)^2], harmonics [E,(L_edge+1)^2], gates [E,P*C] or [E,P,C] (operators.py:310-340).
+        The operands are saved for the backward as passed, in both layouts: changed in place before it, it raises."""
         _tp_coverage(self.tp, self.input_lmax, self.edge_lmax)
         _eager(features)
         if features.ndim != 2:

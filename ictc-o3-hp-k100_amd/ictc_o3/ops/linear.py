@@ -69,7 +69,7 @@ class SpeciesOrder:
 
     def __init__(self, species: torch.Tensor, S: int):
         from ictc_o3.ops.tensor_product import Csr
-        csr = Csr(species.contiguous(), S)   # ictc_csr_build: stable radix sort over the species bits
+        csr = Csr(species.contiguous(), S)   # ictc_csr_build: a stable sort
         self.csr, self.perm, self.off = csr, csr.order, csr.ptr
         self.S, self.N = S, species.shape[0]
 
