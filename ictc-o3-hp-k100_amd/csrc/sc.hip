@@ -224,6 +224,9 @@ int64_t ictc_sc_table_workspace_bytes(int lmax, int target_lmax, int correlation
   Shape sh;
   int64_t floats;
   if (check_tab(lmax, target_lmax, correlation, channels, num_species, nodes, weight_gradients, &sh, &floats)) return -1;
+  // a workspace made for the most nodes and species serves fewer
+  const int64_t pairs = dispatch_tab(lmax, target_lmax, correlation, 0, TabPairs{});
+  if (weight_gradients) floats = ictc::sc::tab_most_chunks(nodes, pairs, channels, num_species) * pairs * channels;
   return floats * (int64_t)sizeof(float);
 }
 

@@ -11,6 +11,8 @@
 // instead of one per term), adds the chunks in order, and contracts pairs with weights once at the end.
 // Deterministic: every sum runs in a fixed order.
 #pragma once
+#include <algorithm>
+
 #include "sc_kernels.h"
 
 namespace ictc {
@@ -31,15 +33,22 @@ struct TabArgs {
 
 // Nodes per weight-gradient chunk (at least 32): the chunks, channel groups and pair blocks together make about
 // kTabDwWaves waves.
-inline int64_t tab_chunk(int64_t nodes, int64_t pairs, int channels) {
+inline int64_t tab_chunks(int64_t pairs, int channels) {
   const int64_t waves = ((channels + 63) / 64) * ((pairs + kPairBlock - 1) / kPairBlock);
-  const int64_t chunks = (kTabDwWaves + waves - 1) / waves;
+  return (kTabDwWaves + waves - 1) / waves;
+}
+inline int64_t tab_chunk(int64_t nodes, int64_t pairs, int channels) {
+  const int64_t chunks = tab_chunks(pairs, channels);
   const int64_t c = ((nodes + chunks - 1) / chunks + 31) / 32 * 32;
   return c < 32 ? 32 : c;
 }
 inline int64_t tab_max_chunks(int64_t nodes, int64_t pairs, int channels, int species) {
   const int64_t c = tab_chunk(nodes, pairs, channels);
   return (nodes + c - 1) / c + species;
+}
+// As many or more, and never fewer for more nodes (the chunks of a call fall where their nodes step up by 32).
+inline int64_t tab_most_chunks(int64_t nodes, int64_t pairs, int channels, int species) {
+  return std::min((nodes + 31) / 32, tab_chunks(pairs, channels)) + species;
 }
 inline int64_t tab_floats(int64_t pairs, int channels, int species) {
   return (int64_t)species * ((channels + 63) / 64) * pairs * 64;

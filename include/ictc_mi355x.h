@@ -712,7 +712,8 @@ int ictc_sc_bwd_w_jvp(int lmax, int target_lmax, int correlation, int channels, 
  *          with grad and tangent Hess_x(grad . out) h;
  *   bwd_w: dW as ictc_sc_bwd_w, with tangent as ictc_sc_bwd_w_jvp.
  * workspace: ictc_sc_table_workspace_bytes(..., weight_gradients = 0 for apply, 1
- * for bwd_w) bytes (-1: no table form or an argument out of range).            */
+ * for bwd_w) bytes (-1: no table form or an argument out of range); the size for the
+ * most nodes and species serves fewer.                                          */
 int ictc_sc_table_pairs(int lmax, int target_lmax, int correlation);
 int64_t ictc_sc_table_workspace_bytes(int lmax, int target_lmax, int correlation, int channels, int64_t nodes,
                                       int num_species, int weight_gradients);

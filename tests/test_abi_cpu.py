@@ -206,6 +206,16 @@ def test_csr_workspace_covers_smaller_lists():
     assert all(a <= b for r, s in zip(size, size[1:]) for a, b in zip(r, s))
 
 
+@pytest.mark.parametrize("weight_gradients", [0, 1])
+def test_table_workspace_covers_fewer_nodes_and_species(weight_gradients):
+    from ictc_o3 import _native
+    f = _native.lib().ictc_sc_table_workspace_bytes
+    for shape in ((3, 2, 3, 128), (3, 1, 3, 64), (2, 2, 3, 64)):
+        size = [[f(*shape, N, S, weight_gradients) for S in (1, 2, 90)] for N in (*range(1, 40000, 61), 10 ** 6)]
+        assert all(0 < a <= b for row in size for a, b in zip(row, row[1:]))
+        assert all(a <= b for r, s in zip(size, size[1:]) for a, b in zip(r, s))
+
+
 def test_species_entry_points_host_checks():
     """Argument checks of the species-sorted self connection and its weight gradient (no device work)."""
     from ictc_o3 import _native
