@@ -257,10 +257,10 @@ def _weight_operand(w, transpose=False):
     slot = id(base)
     entry = _operand_cache.get(slot)
     if entry is None or entry[0]() is not base:
-        def drop(ref):
-            held = _operand_cache.get(slot)
+        def drop(ref, cache=_operand_cache):   # (bound here: it may run as the interpreter ends)
+            held = cache.get(slot)
             if held is not None and held[0] is ref:
-                del _operand_cache[slot]
+                del cache[slot]
         entry = (weakref.ref(base, drop), {})
         _operand_cache[slot] = entry
     views = entry[1]

@@ -2,6 +2,7 @@
 through .data (as weight averaging does), a new storage, and a weight kept in transposed storage.  The reference is
 the autograd route of a fresh copy of the model, which has kept nothing from earlier calls."""
 import copy
+import gc
 
 import pytest
 import torch
@@ -98,6 +99,7 @@ def test_calls_keep_no_copies_of_weights(device):
     model, args = _model(device, 3), _system(device, 3)
     energy_and_forces(model, *args)
     linear._operand_cache.clear()
+    gc.collect()
     torch.cuda.synchronize()
     held = torch.cuda.memory_allocated()
     for _ in range(3):

@@ -22,12 +22,12 @@ def test_memo_replaced_between_reads(monkeypatch):
             if i == 1:      # after the key has been compared
                 lin._order_memo = other
             return tuple.__getitem__(self, i)
+    monkeypatch.setattr(lin, "_order_memo", None)
     lin.species_order(b, 3)
     other = lin._order_memo
     first = lin.species_order(a, 3)
     lin._order_memo = Replaced(lin._order_memo)
     assert lin.species_order(a, 3) is first and first.species is a
-    monkeypatch.setattr(lin, "_order_memo", None)
 
 
 @pytest.mark.gpu
