@@ -99,6 +99,19 @@ def _use_table(spec, N, weights=False) -> bool:
     return waves >= (_TABLE_WEIGHT_WAVES if weights else _TABLE_WAVES[spec.lmax]) and N >= per * spec.num_species
 
 
+# A call that has to make the species order for the tables alone pays its three launches besides.  Whole calls, us, per
+# node -> table, forward / forward and feature gradient: (3,1), 64 channels, 4,096 nodes 35 -> 48 / 138 -> 181, 8,192
+# 71 -> 48 / 160 -> 179, 12,000 105 -> 52 / 236 -> 182; (2,2), 64 channels, 32,768 nodes 51 -> 55 / 156 -> 198, 65,536
+# 113 -> 105 / 271 -> 229; (3,2), 4,096 nodes 95 -> 56 / 213 -> 194.
+_TABLE_OWN_ORDER_WAVES = {(3, 1): 10240, (2, 2): 65536}
+
+
+def _order_pays(spec, N, holder) -> bool:
+    """Whether the species order is there or made anyway, or the tables save more than it costs."""
+    return (holder.ordered(spec.channels)
+            or N * ((spec.channels + 63) // 64) >= _TABLE_OWN_ORDER_WAVES.get((spec.lmax, spec.target_lmax), 0))
+
+
 def _table_raw(spec, x, csr, ws, go=None, tangent=None):
     """SC(x), its tangent, or with go the feature gradient or its tangent, on the coefficient tables."""
     N = x.shape[0]
@@ -113,7 +126,7 @@ def _table_raw(spec, x, csr, ws, go=None, tangent=None):
 
 
 def _fwd_raw(spec, x, species, ws, tangent=None, holder=None):
-    if holder is not None and _use_table(spec, x.shape[0]):
+    if holder is not None and _use_table(spec, x.shape[0]) and _order_pays(spec, x.shape[0], holder):
         return _table_raw(spec, x, holder.species_csr().csr, ws, tangent=tangent)
     out = x.new_empty(x.shape[0], spec.no * spec.channels)
     if tangent is None:
@@ -126,7 +139,7 @@ def _fwd_raw(spec, x, species, ws, tangent=None, holder=None):
 
 
 def _dx_raw(spec, x, species, ws, go, tangent=None, holder=None):
-    if holder is not None and _use_table(spec, x.shape[0]):
+    if holder is not None and _use_table(spec, x.shape[0]) and _order_pays(spec, x.shape[0], holder):
         return _table_raw(spec, x, holder.species_csr().csr, ws, go, tangent)
     dx = torch.empty_like(x)
     if tangent is None:
@@ -233,10 +246,16 @@ class _SCAdjoint(torch.autograd.Function):
 
 class _SpeciesHolder:
     """Lazily built species-sorted node CSR, shared by the adjoints of one forward call (shared=True: the
-    model's order of this step's species tensor, which its self connections use as well)."""
+    model's order of this step's species tensor, which its self connections use as well).  weight_gradients: the
+    call's weights ask for gradients, which are taken in this order."""
 
-    def __init__(self, species, num_species, shared=False):
+    def __init__(self, species, num_species, shared=False, weight_gradients=False):
         self.species, self.num_species, self.shared, self._csr = species, num_species, shared, None
+        self.weight_gradients = weight_gradients
+
+    def ordered(self, channels) -> bool:
+        """Whether the order is there, or made without this contraction (self connections: 64 or 128 channels)."""
+        return self._csr is not None or self.weight_gradients or (self.shared and channels in (64, 128))
 
     def species_csr(self):
         if self._csr is None:
@@ -250,7 +269,8 @@ class _SpeciesHolder:
 
 def symmetric_contraction(x, species, weights: List[torch.Tensor], spec: ScSpec, shared_order=False):
     """x [N, NX*C] packed ir_mul, species [N] int64, weights in spec.slots order -> [N, NO*C] packed ir_mul."""
-    holder = _SpeciesHolder(species, spec.num_species, shared_order)
+    holder = _SpeciesHolder(species, spec.num_species, shared_order,
+                            torch.is_grad_enabled() and any(w.requires_grad for w in weights))
     return _SC.apply(spec, species, holder, x, *weights)
 
 
